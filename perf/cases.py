@@ -280,17 +280,18 @@ def work(case):
 
 # Largest relative error of another correct implementation: bf16 results whose
 # fp32 sums run in another order differ where a sum falls on the other side of
-# a rounding boundary (one bf16 step, 2^-8 of the value). Through the expert
-# block such a step travels on from gate/up, act and down; measured against
-# sums in 64 bits with the same bf16 rounding points: 2e-4 for single
-# products, 1e-3 for expert blocks and the shared expert.
+# a rounding boundary (one bf16 step, at most 2^-7 of the value). Through the
+# expert block such a step travels on from gate/up, act and down. Measured
+# against sums in 64 bits with the same bf16 rounding points: up to 4e-5 for
+# the projections (more where a call has few outputs and one of them steps),
+# 1.5e-4 for the shared expert, 2e-5 to 9e-4 for the expert blocks.
 def tolerance(case):
     kind = case["kind"]
     if kind in ("combine", "convert"):  # fixed order of the sum, whole numbers: the same bits
         return "exact"
     if kind in ("w4", "w8"):
         return {"rel": 1e-3, "max": 0.01}
-    return {"rel": 4e-3}
+    return {"rel": 4e-3 if kind == "experts" else 1e-3}
 
 
 # ---------------------------------------------------------------- the same in 64 bits
