@@ -5,7 +5,8 @@
 //
 // q int8 [K, N] (row k holds the N columns), S bf16 [K/gs, N], x bf16 [M, K].
 //
-// M <= 4: split-K GEMV. A workgroup owns 256 columns (16 chunks of 16 bytes)
+// M <= 4 where the MFMA forms do not take the shape, and one row of a long K:
+// split-K GEMV. A workgroup owns 256 columns (16 chunks of 16 bytes)
 // and a K-slice of 16 L rows: thread (row-lane r = tid/16, chunk tid%16)
 // loads its L rows of 16 columns at once (L = 4, 8 or 16, the most that
 // keeps >= 512 workgroups in the grid and a run inside one scale group). A byte is read as offset binary u = q + 128
@@ -15,8 +16,10 @@
 // Row-lanes are summed in LDS in row-lane order, the K-slices by the last
 // workgroup to arrive, in slice order: deterministic run to run.
 //
-// M > 4: bf16 MFMA (16x16x32) on 64- or 128-row, 64-column output tiles,
-// the operands streaming through an LDS ring of chunks. int8 values are exact in bf16, so the MFMA sums
+// Few rows or few tiles: bf16 MFMA (16x16x32), K split over a workgroup's
+// waves, weights streamed into registers.
+// Else: the same MFMA on 128 x 64 output tiles, the operands streaming
+// through an LDS ring of chunks. int8 values are exact in bf16, so the MFMA sums
 // x * q exactly per product with fp32 accumulation; after each scale group
 // the group's partial sums are scaled by S[g, n] and added to the output
 // accumulators.
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(kThreads) void w8a16_gemv_kernel(const uint16_t* __
   }
 }
 
-// ---------------------------------------------------------------- M > 4: MFMA
+// ---------------------------------------------------------------- many tiles: LDS ring
 //
 // bf16 MFMA 16x16x32 on BM x BN output tiles per workgroup of 4 waves (2 x 2,
 // each (BM/2) x (BN/2): TI x TJ MFMA tiles). K runs in KC-wide chunks (one
@@ -459,6 +462,231 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
     }
 }
 
+// ---------------------------------------------------------------- few tiles: K split over the waves
+//
+// 16 LIVE rows of x (LIVE MFMA row tiles) times 16 F columns per workgroup. The
+// NW waves split K (contiguous runs of 32-k steps) and stream their weights
+// straight into registers in MFMA B-fragment order: lane (i16, kb) reads, for
+// each of its 8 k rows 32 s + 8 kb + i, one 4-byte word, and a byte position of
+// the eight words is the B fragment of that column. F = 4: word i16, all four
+// columns (64-byte row pieces); F = 2: word i16 % 8, columns 2 (i16 / 8) and
+// the next (32-byte pieces, the words read twice from the L1). int8 -> bf16
+// (exact) is one conversion per value and one v_perm per pair; a scale group's
+// MFMA sums are scaled by S[g, n] in fp32 as in the tiled kernel. U steps are
+// loaded as one batch while the previous batch is computed. The waves' partial
+// tiles meet in LDS and are summed in wave order: no second launch, counters
+// or partials in memory, and the same bits every run.
+//
+// What bounds it: not HBM (2048 x 8192 at 7 rows: 7.9 us for 17 MB) but the
+// workgroup's own chain: launch and first load about 4 us, then ~66 VALU and 10
+// load instructions per step and wave, four waves per SIMD. So the grid takes
+// few rows and columns per workgroup while it still fits the CUs at once.
+// Against the 64 x 64 tiles (one chain over all of K per workgroup) it replaces
+// here: 33.5 -> 7.9 us at 7 rows, 33.9 -> 13.2 at 64 (2048 x 8192), 34.0 -> 7.3
+// at 7 rows, 34.1 -> 13.7 at 512 (2048 x 2048). Nontemporal weight loads lose
+// (11.6 us): the two halves of a 128-byte line are read by two workgroups of one
+// XCD and the second then misses.
+template <int LIVE, int NW, int U, int F>
+__global__ __launch_bounds__(64 * NW) void w8a16_skinny_kernel(const uint16_t* __restrict__ x,
+                                                               const int8_t* __restrict__ w,
+                                                               const uint16_t* __restrict__ s,
+                                                               uint16_t* __restrict__ y, int M, int K, int N, int gs) {
+  constexpr int BN = 16 * F, ROWS = 16 * LIVE;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  float* red = reinterpret_cast<float*>(lds);  // [NW][ROWS][BN]
+  const int nrg = (M + ROWS - 1) / ROWS;
+  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  if (tile >= nrg * ((N + BN - 1) / BN)) return;
+  const int m0 = (tile % nrg) * ROWS, n0 = (tile / nrg) * BN;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i16 = lane & 15, kb = lane >> 4;
+  const int nsteps = K / kBK, spg = gs / kBK;  // steps per scale group
+  const int per = (nsteps + NW - 1) / NW;
+  const int s0 = min(nsteps, wave * per), s1 = min(nsteps, s0 + per);
+  // columns past N read column 0 (never stored), rows past M the last row
+  const int cl = F == 4 ? 4 * i16 : 4 * (i16 & 7);  // the lane's word: tile columns cl .. cl + 3
+  const int lc = F == 4 ? cl : cl + 2 * (i16 >> 3);  // its first column: lc .. lc + F - 1
+  const int c0 = n0 + cl < N ? n0 + cl : 0;
+  // buffer resources: per-lane offsets fixed for the whole loop, a scalar
+  // offset per step, every access bounded by its tensor
+  constexpr int kRsrcWord3 = 0x00020000;
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, M * K * 2, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, K * N, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_s =
+      __builtin_amdgcn_make_buffer_rsrc((void*)s, (short)0, (K / gs) * N * 2, kRsrcWord3);
+  const int boff = 8 * kb * N + c0;
+  const int sh = 16 * (i16 >> 3);  // F = 2: this lane's half of the word
+  int aoff[LIVE];
+#pragma unroll
+  for (int t = 0; t < LIVE; ++t) aoff[t] = 2 * (min(m0 + 16 * t + i16, M - 1) * K + 8 * kb);
+
+  f32x4_v acc[LIVE][F], accg[LIVE][F];
+#pragma unroll
+  for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+    for (int f = 0; f < F; ++f) acc[t][f] = accg[t][f] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+
+  struct Block {
+    uint32_t b[U][8];
+    uint4 a[U][LIVE];
+    uint2 sc[U];
+  };
+  // the load position: a step, its scale group's row and the group's steps
+  // left (counted, not divided); steps past the wave's last re-read it (their
+  // results are not used)
+  int lq = s0, lrow = 0, lleft = 0, cleft = 0;
+  auto load_block = [&](Block& v) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        v.b[u][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc_b, boff, (lq * kBK + i) * N, 0);
+#pragma unroll
+      for (int t = 0; t < LIVE; ++t)
+        v.a[u][t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, aoff[t], lq * kBK * 2, 0));
+      v.sc[u] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rsrc_s, 2 * c0, lrow, 0));
+      if (lq + 1 < s1) {
+        ++lq;
+        if (--lleft == 0) {
+          lleft = spg;
+          lrow += 2 * N;
+        }
+      }
+    }
+  };
+  auto compute = [&](int st, const Block& v) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = st + u;
+      if (q >= s1) break;
+      uint32_t b[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) b[i] = F == 4 ? v.b[u][i] : v.b[u][i] >> sh;
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        uint32_t p[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float lo = (float)(int)(int8_t)(b[2 * i] >> (8 * f));
+          const float hi = (float)(int)(int8_t)(b[2 * i + 1] >> (8 * f));
+          p[i] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+        }
+        const bf16x8_v bf = __builtin_bit_cast(bf16x8_v, make_uint4(p[0], p[1], p[2], p[3]));
+#pragma unroll
+        for (int t = 0; t < LIVE; ++t)
+          accg[t][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_v, v.a[u][t]), bf, accg[t][f], 0, 0, 0);
+      }
+      if (--cleft == 0 || q + 1 == s1) {
+        cleft = spg;
+        const uint32_t s01 = (F == 4 || i16 < 8) ? v.sc[u].x : v.sc[u].y;
+        const float sc[4] = {bf16_to_f32(s01 & 0xffffu), bf16_to_f32(s01 >> 16), bf16_to_f32(v.sc[u].y & 0xffffu),
+                             bf16_to_f32(v.sc[u].y >> 16)};
+#pragma unroll
+        for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+          for (int f = 0; f < F; ++f) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][f][r] = __builtin_fmaf(accg[t][f][r], sc[f], acc[t][f][r]);
+            accg[t][f] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+          }
+      }
+    }
+  };
+  if (s0 < s1) {
+    const int g0 = s0 / spg;
+    lrow = g0 * N * 2;
+    lleft = cleft = spg - (s0 - g0 * spg);
+    Block v0, v1;
+    load_block(v0);
+    for (int st = s0; st < s1; st += 2 * U) {
+      if (st + U < s1) load_block(v1);
+      compute(st, v0);
+      if (st + 2 * U < s1) load_block(v0);
+      if (st + U < s1) compute(st + U, v1);
+    }
+  }
+  // lane holds, for each row tile, rows 4 kb + r of its F columns
+#pragma unroll
+  for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      float* dst = red + ((size_t)wave * ROWS + 16 * t + 4 * kb + r) * BN + lc;
+      if constexpr (F == 4) *reinterpret_cast<float4*>(dst) = make_float4(acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]);
+      else *reinterpret_cast<float2*>(dst) = make_float2(acc[t][0][r], acc[t][1][r]);
+    }
+  __syncthreads();
+  for (int p = tid; p < min(ROWS, M - m0) * BN / 4; p += 64 * NW) {
+    const int row = p / (BN / 4), c = 4 * (p % (BN / 4));
+    float4 a = *reinterpret_cast<const float4*>(red + row * BN + c);
+#pragma unroll
+    for (int q = 1; q < NW; ++q) {
+      const float4 b = *reinterpret_cast<const float4*>(red + ((size_t)q * ROWS + row) * BN + c);
+      a.x += b.x;
+      a.y += b.y;
+      a.z += b.z;
+      a.w += b.w;
+    }
+    if (n0 + c < N)
+      *reinterpret_cast<uint2*>(y + (size_t)(m0 + row) * N + n0 + c) =
+          make_uint2(f32_to_bf16(a.x) | (f32_to_bf16(a.y) << 16), f32_to_bf16(a.z) | (f32_to_bf16(a.w) << 16));
+  }
+}
+
+template <int LIVE, int NW, int U, int F>
+int launch_w8_skinny(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs,
+                     hipStream_t stream) {
+  constexpr int kLds = NW * 16 * LIVE * 16 * F * 4;
+  int dev = 0;
+  hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return (int)err;
+  if (dev < 0 || dev >= 64) return QMOE_EINVAL;
+  static bool attr_set[64] = {};
+  if (!attr_set[dev]) {
+    err = hipFuncSetAttribute((const void*)w8a16_skinny_kernel<LIVE, NW, U, F>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (err != hipSuccess) return (int)err;
+    attr_set[dev] = true;
+  }
+  const long tiles = (long)host_ceil_div(M, 16 * LIVE) * host_ceil_div(N, 16 * F);
+  const long blocks = (tiles + 7) / 8 * 8;  // whole XCD rounds (extra blocks exit)
+  if (blocks > 0x7fffffffL) return QMOE_EINVAL;
+  hipLaunchKernelGGL((w8a16_skinny_kernel<LIVE, NW, U, F>), dim3((unsigned)blocks), dim3(64 * NW), kLds, stream,
+                     (const uint16_t*)x, (const int8_t*)w, (const uint16_t*)scale, (uint16_t*)y, M, K, N, gs);
+  return (int)hipGetLastError();
+}
+
+bool w8_mfma_ok(const void* x, const void* w, int M, int K, int N, int gs) {
+  return M >= 1 && K >= kBK && K % kBK == 0 && N >= 16 && N % 16 == 0 && gs >= kBK && gs % kBK == 0 && K % gs == 0 &&
+         ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && (long)M * K * 2 < 0x80000000L &&
+         (long)K * N < 0x80000000L;
+}
+
+// The skinny kernel's tile: the fewest row tiles per workgroup whose grid
+// still runs at once (a workgroup's 8 or 16 waves take a CU), 32-column tiles
+// where those fit the 256 CUs as well.
+// Few rows and many workgroups win because each workgroup's conversions and x
+// reads, not HBM, set its time: at K = 2048 one, two, three and four row tiles
+// take 7.9, 10.0, 11.6 and 13.2 us with 32 columns, 8.3, 10.6, 11.8 and 13.7
+// with 64, whatever N is (2048 or 8192).
+int launch_w8_few_tiles(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs,
+                        hipStream_t st) {
+  constexpr long kCus = 256;
+  auto groups = [&](int live) { return (long)host_ceil_div(M, 16 * live); };
+  int live = 1;
+  while (live < 4 && groups(live) * host_ceil_div(N, 64) > kCus) ++live;
+  live = host_ceil_div(M, 16 * (int)groups(live));  // no emptier than needed
+  if (groups(live) * host_ceil_div(N, 32) <= kCus) {
+    if (live == 1) return launch_w8_skinny<1, 16, 1, 2>(x, w, scale, y, M, K, N, gs, st);
+    if (live == 2) return launch_w8_skinny<2, 16, 2, 2>(x, w, scale, y, M, K, N, gs, st);
+    if (live == 3) return launch_w8_skinny<3, 8, 2, 2>(x, w, scale, y, M, K, N, gs, st);
+    return launch_w8_skinny<4, 8, 2, 2>(x, w, scale, y, M, K, N, gs, st);
+  }
+  if (live == 1) return launch_w8_skinny<1, 16, 2, 4>(x, w, scale, y, M, K, N, gs, st);
+  if (live == 2) return launch_w8_skinny<2, 16, 1, 4>(x, w, scale, y, M, K, N, gs, st);
+  if (live == 3) return launch_w8_skinny<3, 8, 1, 4>(x, w, scale, y, M, K, N, gs, st);
+  return launch_w8_skinny<4, 8, 1, 4>(x, w, scale, y, M, K, N, gs, st);
+}
+
 template <class T>
 int launch_w8_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs,
                    hipStream_t stream) {
@@ -506,6 +734,14 @@ int qmoe_w8a16_gemv(const void* x, const void* w, const void* scale, void* y, in
   if (M < 1 || M > 4 || K < 4 || (K % 4) || N < 16 || (N % 16) || group_size < 4 || (group_size % 4) ||
       (K % group_size) || host_ceil_div(N, kTileCols) >= QMOE_DECODE_MAILBOX_BASE - 1)
     return QMOE_EINVAL;
+  // The skinny MFMA kernel where it takes the shape: its 16 waves share K, so
+  // it needs no second reduction through memory. Two to four rows: 8.3 against
+  // 11.7 to 16.5 us (2048 x 8192), 10.5 against 19.2 (three rows, 4096 x 512).
+  // One row: faster up to 2560 rows of K (2048 x 8192 7.5 against 9.3 us,
+  // 2560 x 8192 8.7 against 10.7), slower above, where each wave's run of K is
+  // long (4096 x 512 10.0 against 8.5, 4096 x 8192 14.7 against 13.5).
+  if ((M > 1 || K <= 2560) && w8_mfma_ok(x, w, M, K, N, group_size))
+    return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, (hipStream_t)stream);
   const int L = w8_rows_per_thread(K, N, group_size);
   const int nslices = host_ceil_div(K, kRowLanes * L);
   if (nslices > 1 && workspace_bytes < qmoe_w8a16_gemv_workspace(M, K, N)) return QMOE_EWORKSPACE;
@@ -529,18 +765,17 @@ int qmoe_w8a16_gemv(const void* x, const void* w, const void* scale, void* y, in
 
 int qmoe_w8a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,
                          int group_size, void* stream) {
-  if (M < 1 || K < kBK || (K % kBK) || N < 16 || (N % 16) || group_size < kBK || (group_size % kBK) ||
-      (K % group_size) || ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
-      (long)M * K * 2 >= 0x80000000L || (long)K * N >= 0x80000000L)
-    return QMOE_EINVAL;
+  if (!w8_mfma_ok(x, w, M, K, N, group_size)) return QMOE_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  // 128 x 64 tiles where they still give every CU a workgroup (64-k chunks
-  // when the group size allows: twice the MFMA work per barrier), else 64 x 64
+  // 128 x 64 tiles (64-k chunks when the group size allows: twice the MFMA work
+  // per barrier) above 256 rows where they still give every CU a workgroup,
+  // else the skinny kernel. At 2048 x 8192 the tiles take 28.5 us for 129 to
+  // 256 rows, the skinny kernel 20.1 to 24.9; at 512 rows 39.1 against 46.5.
   const long tiles128 = (long)((M + 127) / 128) * ((N + 63) / 64);
-  if (tiles128 >= 256 && group_size % 64 == 0 && K % 64 == 0)
+  if (M <= 256 || tiles128 < 256) return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, st);
+  if (group_size % 64 == 0 && K % 64 == 0)
     return launch_w8_mfma<W8Tile<128, 64, 64, 3>>(x, w, scale, y, M, K, N, group_size, st);
-  if (tiles128 >= 256) return launch_w8_mfma<W8Tile<128, 64, 32, 4>>(x, w, scale, y, M, K, N, group_size, st);
-  return launch_w8_mfma<W8Tile<64, 64, 32, 4>>(x, w, scale, y, M, K, N, group_size, st);
+  return launch_w8_mfma<W8Tile<128, 64, 32, 4>>(x, w, scale, y, M, K, N, group_size, st);
 }
 
 }  // extern "C"

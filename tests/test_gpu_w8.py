@@ -52,6 +52,26 @@ def test_w8a16_gemm_wide_tiles(device, M, K, N, gs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 16, 17, 33, 49, 64, 65, 200, 257])
+@pytest.mark.parametrize("K,N,gs", [(32, 16, 32), (480, 1040, 96), (1088, 80, 64), (2560, 48, 32), (544, 8208, 544)])
+def test_w8a16_few_tiles(device, M, K, N, gs):
+    """K split over a workgroup's waves: fewer steps than waves, runs that cut
+    scale groups, ragged rows and columns, both column widths, and scales that
+    start off a 16-byte boundary."""
+    from qmoe import weight_quant_batchmatmul
+    log(f"w8a16 few tiles M={M} K={K} N={N} gs={gs}")
+    x, q, S = w8_case(M, K, N, gs, M + 5 * K + N)
+    sd = torch.empty(K // gs * N + 1, dtype=torch.bfloat16, device=device)[1:].view(K // gs, N)
+    sd.copy_(to_dev(S, device))
+    xd, qd = to_dev(x, device), to_dev(q, device)
+    y = weight_quant_batchmatmul(xd, qd, sd, antiquant_group_size=gs)
+    y2 = weight_quant_batchmatmul(xd, qd, sd, antiquant_group_size=gs)
+    torch.cuda.synchronize()
+    check(bits(y), x, q, S, gs, f"w8a16 few tiles M={M}")
+    assert np.array_equal(bits(y), bits(y2))
+
+
+@pytest.mark.gpu
 def test_w8a16_small_group_gemv(device):
     """gs = 8 (a 4-row run per thread stays in one group) on the GEMV path."""
     from qmoe import weight_quant_batchmatmul
