@@ -5,8 +5,8 @@
 //
 // q int8 [K, N] (row k holds the N columns), S bf16 [K/gs, N], x bf16 [M, K].
 //
-// M <= 4 where the MFMA forms do not take the shape, and one row of a long K:
-// split-K GEMV. A workgroup owns 256 columns (16 chunks of 16 bytes)
+// One row, and up to four where the MFMA forms do not take the shape: split-K
+// GEMV. A workgroup owns 256 columns (16 chunks of 16 bytes)
 // and a K-slice of 16 L rows: thread (row-lane r = tid/16, chunk tid%16)
 // loads its L rows of 16 columns at once (L = 4, 8 or 16, the most that
 // keeps >= 512 workgroups in the grid and a run inside one scale group). A byte is read as offset binary u = q + 128
@@ -734,13 +734,11 @@ int qmoe_w8a16_gemv(const void* x, const void* w, const void* scale, void* y, in
   if (M < 1 || M > 4 || K < 4 || (K % 4) || N < 16 || (N % 16) || group_size < 4 || (group_size % 4) ||
       (K % group_size) || host_ceil_div(N, kTileCols) >= QMOE_DECODE_MAILBOX_BASE - 1)
     return QMOE_EINVAL;
-  // The skinny MFMA kernel where it takes the shape: its 16 waves share K, so
-  // it needs no second reduction through memory. Two to four rows: 8.3 against
-  // 11.7 to 16.5 us (2048 x 8192), 10.5 against 19.2 (three rows, 4096 x 512).
-  // One row: faster up to 2560 rows of K (2048 x 8192 7.5 against 9.3 us,
-  // 2560 x 8192 8.7 against 10.7), slower above, where each wave's run of K is
-  // long (4096 x 512 10.0 against 8.5, 4096 x 8192 14.7 against 13.5).
-  if ((M > 1 || K <= 2560) && w8_mfma_ok(x, w, M, K, N, group_size))
+  // Two to four rows: the skinny MFMA kernel where it takes the shape (its waves
+  // share K, so it needs no second reduction through memory): 8.3 against 11.7
+  // to 16.5 us (2048 x 8192), 10.5 against 19.2 (three rows, 4096 x 512). One
+  // row stays here: from cold weights 9.0 us against 9.75 (2048 x 8192).
+  if (M > 1 && w8_mfma_ok(x, w, M, K, N, group_size))
     return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, (hipStream_t)stream);
   const int L = w8_rows_per_thread(K, N, group_size);
   const int nslices = host_ceil_div(K, kRowLanes * L);
