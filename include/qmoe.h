@@ -56,6 +56,12 @@ int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
  *      tile_expert/tile_row0/tile_rows [mtiles_max], tile_count [1]) is built
  *      on the GPU by qmoe_tiles_from_ends or qmoe_route_group. */
 int qmoe_gemm_tile_rows(void);
+/* Row-tile sizes the grouped GEMMs take: qmoe_gemm_tile_rows() or 12 (the
+ * few-rows kernel, for shapes these return it for). The size to build the
+ * tables with for R rows over E experts: one GEMM [K, N], or the expert block
+ * (both GEMMs, hidden H, width MI); pass it on as tile_rows_max. */
+int qmoe_gemm_tile_rows_for(int R, int E, int K, int N, int gs);
+int qmoe_moe_tile_rows(int R, int E, int H, int MI, int gs_gu, int gs_dn);
 int qmoe_max_row_tiles(int R, int E, int BM);
 int qmoe_tiles_from_ends(const void* ends_i64, int E, int R, int BM, void* tile_expert, void* tile_row0,
                          void* tile_rows, void* tile_count, void* stream);
@@ -71,6 +77,12 @@ int qmoe_grouped_gemm(const void* x, int R, int K, int N, int E, int gs, const v
                       const void* tile_expert, const void* tile_row0, const void* tile_rows,
                       const void* tile_count, int mtiles_max, void* y, void* workspace, size_t workspace_bytes,
                       void* stream);
+/* The same with tables whose tiles hold at most tile_rows_max rows: one of the
+ * sizes above (qmoe_grouped_gemm takes qmoe_gemm_tile_rows()). */
+int qmoe_grouped_gemm_rows(const void* x, int R, int K, int N, int E, int gs, const void* w, const void* scale,
+                           int tile_rows_max, const void* tile_expert, const void* tile_row0, const void* tile_rows,
+                           const void* tile_count, int mtiles_max, void* y, void* workspace, size_t workspace_bytes,
+                           void* stream);
 
 /* ---- Router: probs = softmax(fp32 logits); top-k by (logit desc, id asc);
  *      w = bf16(p / sum of selected p). fnx/engine.py:1810-1813.
@@ -239,6 +251,13 @@ int qmoe_moe_experts_grouped(const void* x, int T, int H, int MI, int E, int k, 
                              const void* tile_row0, const void* tile_rows, const void* tile_count,
                              int mtiles_max, const void* shared, void* out, void* workspace,
                              size_t workspace_bytes, void* stream);
+/* The same with tables whose tiles hold at most tile_rows_max rows. */
+int qmoe_moe_experts_grouped_rows(const void* x, int T, int H, int MI, int E, int k, const void* wts,
+                                  const void* order, const void* gu_w, const void* gu_s, int gs_gu,
+                                  const void* dn_w, const void* dn_s, int gs_dn, int tile_rows_max,
+                                  const void* tile_expert, const void* tile_row0, const void* tile_rows,
+                                  const void* tile_count, int mtiles_max, const void* shared, void* out,
+                                  void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- fnx_gather_pair (kernels/expert_gather/gather.cpp:24-27, wrapper
  *      fnx/expert_gather.py:9-31): ow[kk, j*N/8 + c] = w4[ids[j], kk, c],

@@ -27,14 +27,6 @@ typedef float f32x4_v __attribute__((ext_vector_type(4)));
 constexpr int kThreads = 256;
 constexpr int BK = 32;  // k per MFMA step
 
-// s_waitcnt with vmcnt <= N and lgkmcnt == 0 (gfx9 encoding: vmcnt bits
-// [3:0] and [15:14], expcnt [6:4] left at 7).
-template <int N>
-QMOE_DEV void wait_vm_lgkm0() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4));
-}
-
 template <int BM_, int BN_, int KC_, int RING_>
 struct Bf16Tile {
   static constexpr int BM = BM_, BN = BN_, KC = KC_, RING = RING_;

@@ -42,6 +42,7 @@
 // scattered to token-major rows for the ordered slot reduction.
 #include "qmoe_common.h"
 #include "qmoe.h"
+#include "w4_few_rows.h"
 
 namespace {
 
@@ -49,8 +50,6 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;    // 4 waves; two workgroups per CU, so two waves per SIMD
 constexpr int BM = 128;          // rows per tile
@@ -90,29 +89,8 @@ struct GemmArgs {
 
 QMOE_DEV half2_t as_h2(uint32_t v) { return __builtin_bit_cast(half2_t, v); }
 QMOE_DEV uint32_t h2_bits(half2_t v) { return __builtin_bit_cast(uint32_t, v); }
-QMOE_DEV uint32_t pk_rtz(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
-}
-// bf16 pair (RNE, hardware conversion; finite values round exactly like f32_to_bf16)
-QMOE_DEV uint32_t pk_bf16(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t));
-}
 QMOE_DEV float bf16_lo(uint32_t v) { return __uint_as_float(v << 16); }
 QMOE_DEV float bf16_hi(uint32_t v) { return __uint_as_float(v & 0xffff0000u); }
-
-// exponent that brings a magnitude with bf16 biased exponent eb into [2^t, 2^(t+1)), t = target - 127
-QMOE_DEV int exp_to(uint32_t max_abs_bits, int target_biased) {
-  const int eb = (int)(max_abs_bits >> 7) & 0xff;
-  return eb == 0 ? 0 : target_biased - eb;
-}
-
-// s_waitcnt with vmcnt <= N and lgkmcnt == 0 (gfx9 encoding: vmcnt bits
-// [3:0] and [15:14], expcnt [6:4] left at 7).
-template <int N>
-QMOE_DEV void wait_vm_lgkm0() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4));
-}
 
 // LDS accesses the compiler does not track. The compiler cannot tell which
 // LDS bytes an in-flight global->LDS DMA writes, so it would wait for every
@@ -144,14 +122,6 @@ QMOE_DEV void lds_write4_settled(void* p, uint32_t v) {
 }
 QMOE_DEV void lds_max4_settled(void* p, uint32_t v) {
   asm volatile("ds_max_u32 %0, %1" ::"v"(lds_addr(p)), "v"(v) : "memory");
-}
-
-// Workgroup barrier without a memory fence: the caller has already waited
-// for the memory operations the barrier must order (a fence here would also
-// wait for the prefetches still in flight).
-QMOE_DEV void barrier_no_fence() {
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 // A constant held in a VGPR the compiler cannot see through, so that the
@@ -816,19 +786,39 @@ extern "C" {
 
 int qmoe_gemm_tile_rows(void) { return BM; }
 
+// The few-rows kernel up to five rows per expert on average: 2560/640 g64, 512
+// experts, 128 / 256 tokens 303 / 327 us per block against 342 / 363, 3072/768
+// 256 tokens 427 against 487; at 512 tokens (ten rows) 543 against 506.
+int qmoe_gemm_tile_rows_for(int R, int E, int K, int N, int gs) {
+  return (long)R <= 5L * E && w4_few_rows_ok(K, N, gs) ? kFewRowsTile : BM;
+}
+
+int qmoe_moe_tile_rows(int R, int E, int H, int MI, int gs_gu, int gs_dn) {
+  return max(qmoe_gemm_tile_rows_for(R, E, H, 2 * MI, gs_gu), qmoe_gemm_tile_rows_for(R, E, MI, H, gs_dn));
+}
+
 size_t qmoe_grouped_gemm_workspace(int R, int K) { return plain_ws(R > 0 ? R : 1, K); }
 
-int qmoe_grouped_gemm(const void* x, int R, int K, int N, int E, int gs, const void* w, const void* scale,
-                      const void* tile_expert, const void* tile_row0, const void* tile_rows,
-                      const void* tile_count, int mtiles_max, void* y, void* workspace, size_t workspace_bytes,
-                      void* stream) {
+int qmoe_grouped_gemm_rows(const void* x, int R, int K, int N, int E, int gs, const void* w, const void* scale,
+                           int tile_rows_max, const void* tile_expert, const void* tile_row0, const void* tile_rows,
+                           const void* tile_count, int mtiles_max, void* y, void* workspace, size_t workspace_bytes,
+                           void* stream) {
   if (R < 0 || E < 1 || !gemm_shape_ok(K, N, gs) || !aligned16(x) || !aligned16(y) || !aligned16(scale) ||
-      !aligned16(workspace) || tile_expert == nullptr)
+      !aligned16(workspace) || tile_expert == nullptr || (tile_rows_max != BM && tile_rows_max != kFewRowsTile) ||
+      (tile_rows_max != BM && !w4_few_rows_ok(K, N, gs)))
     return QMOE_EINVAL;
   if (R == 0) return 0;
   if (workspace_bytes < qmoe_grouped_gemm_workspace(R, K)) return QMOE_EWORKSPACE;
   if (!buffer_extent_ok((size_t)R * K * 2) || !buffer_extent_ok((size_t)K * N / 2)) return QMOE_EINVAL;
   hipStream_t st = (hipStream_t)stream;
+  if (tile_rows_max != BM) {
+    FewRowsArgs f{};
+    f.x = (const uint16_t*)x; f.topk = 1; f.w = (const uint32_t*)w; f.s = (const uint16_t*)scale;
+    f.K = K; f.N = N; f.gs = gs; f.tile_expert = (const int*)tile_expert; f.tile_row0 = (const int*)tile_row0;
+    f.tile_rows = (const int*)tile_rows; f.tile_count = (const int*)tile_count; f.mtiles_max = mtiles_max; f.R = R;
+    f.y = (uint16_t*)y; f.ldy = N;
+    return launch_w4_few_rows(0, f, st);
+  }
   _Float16* x16 = (_Float16*)workspace;
   int* rexp = (int*)((char*)workspace + align256((size_t)R * K * 2));
   int rc = launch_rows_to_f16(x, R, K, nullptr, rexp, x16, nullptr, 0, st);
@@ -842,6 +832,14 @@ int qmoe_grouped_gemm(const void* x, int R, int K, int N, int E, int gs, const v
   return launch_gemm<0>(a, mtiles_max, st);
 }
 
+int qmoe_grouped_gemm(const void* x, int R, int K, int N, int E, int gs, const void* w, const void* scale,
+                      const void* tile_expert, const void* tile_row0, const void* tile_rows,
+                      const void* tile_count, int mtiles_max, void* y, void* workspace, size_t workspace_bytes,
+                      void* stream) {
+  return qmoe_grouped_gemm_rows(x, R, K, N, E, gs, w, scale, BM, tile_expert, tile_row0, tile_rows, tile_count,
+                                mtiles_max, y, workspace, workspace_bytes, stream);
+}
+
 size_t qmoe_w4a16_gemm_mfma_workspace(int M, int K) { return plain_ws(M > 0 ? M : 1, K); }
 
 int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs,
@@ -852,6 +850,15 @@ int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
   if (workspace_bytes < qmoe_w4a16_gemm_mfma_workspace(M, K)) return QMOE_EWORKSPACE;
   if (!buffer_extent_ok((size_t)M * K * 2) || !buffer_extent_ok((size_t)K * N / 2)) return QMOE_EINVAL;
   hipStream_t st = (hipStream_t)stream;
+  // The few-rows kernel up to four rounds of its 128-column workgroups on the
+  // CUs: 2048 x 4096 at 64 rows 11.1 against 31.8 us, at 256 21.5 against 45.2,
+  // at 512 40.2 against 45.2.
+  if (w4_few_rows_ok(K, N, gs) && (long)host_ceil_div(M, 16) * host_ceil_div(N, 128) <= 1024) {
+    FewRowsArgs f{};
+    f.x = (const uint16_t*)x; f.topk = 1; f.w = (const uint32_t*)w; f.s = (const uint16_t*)scale;
+    f.K = K; f.N = N; f.gs = gs; f.R = M; f.y = (uint16_t*)y; f.ldy = N;
+    return launch_w4_few_rows_dense(f, st);
+  }
   _Float16* x16 = (_Float16*)workspace;
   int* rexp = (int*)((char*)workspace + align256((size_t)M * K * 2));
   int rc = launch_rows_to_f16(x, M, K, nullptr, rexp, x16, nullptr, 0, st);
@@ -873,15 +880,17 @@ int qmoe_moe_prefill_layout(int T, int k, int H, int MI, size_t* off_act, size_t
   return 0;
 }
 
-int qmoe_moe_experts_grouped(const void* x, int T, int H, int MI, int E, int k, const void* wts,
-                             const void* order, const void* gu_w, const void* gu_s, int gs_gu,
-                             const void* dn_w, const void* dn_s, int gs_dn, const void* tile_expert,
-                             const void* tile_row0, const void* tile_rows, const void* tile_count,
-                             int mtiles_max, const void* shared, void* out, void* workspace,
-                             size_t workspace_bytes, void* stream) {
+int qmoe_moe_experts_grouped_rows(const void* x, int T, int H, int MI, int E, int k, const void* wts,
+                                  const void* order, const void* gu_w, const void* gu_s, int gs_gu,
+                                  const void* dn_w, const void* dn_s, int gs_dn, int tile_rows_max,
+                                  const void* tile_expert, const void* tile_row0, const void* tile_rows,
+                                  const void* tile_count, int mtiles_max, const void* shared, void* out,
+                                  void* workspace, size_t workspace_bytes, void* stream) {
   if (T < 1 || k < 1 || k > QMOE_KMAX || E < 1 || !gemm_shape_ok(H, 2 * MI, gs_gu) || !gemm_shape_ok(MI, H, gs_dn) ||
       !aligned16(x) || !aligned16(out) || !aligned16(gu_s) || !aligned16(dn_s) || !aligned16(workspace) ||
-      (shared != nullptr && !aligned16(shared)) || tile_expert == nullptr)
+      (shared != nullptr && !aligned16(shared)) || tile_expert == nullptr ||
+      (tile_rows_max != BM && tile_rows_max != kFewRowsTile) ||
+      (tile_rows_max != BM && (!w4_few_rows_ok(H, 2 * MI, gs_gu) || !w4_few_rows_ok(MI, H, gs_dn))))
     return QMOE_EINVAL;
   const PrefillLayout l = prefill_layout(T, k, H, MI);
   if (workspace_bytes < l.total) return QMOE_EWORKSPACE;
@@ -898,30 +907,57 @@ int qmoe_moe_experts_grouped(const void* x, int T, int H, int MI, int E, int k, 
   uint32_t* rmax = (uint32_t*)(ws + l.rmax);
   int* rexp_a = (int*)(ws + l.rexp_a);
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_rows_to_f16(x, T, H, nullptr, rexp_x, x16, rmax, R, st);
-  if (rc) return rc;
-  GemmArgs a{};
-  a.a16 = x16; a.lda = H; a.a_bytes = (uint32_t)((size_t)T * H * 2); a.perm = (const int64_t*)order; a.topk = k; a.rexp = rexp_x; a.rmax_out = rmax;
-  a.w = (const uint32_t*)gu_w; a.s = (const uint16_t*)gu_s; a.K = H; a.N = 2 * MI; a.gs = gs_gu;
-  a.tile_expert = (const int*)tile_expert; a.tile_row0 = (const int*)tile_row0;
-  a.tile_rows = (const int*)tile_rows; a.tile_count = (const int*)tile_count; a.R = R;
-  a.n_ntiles = host_ceil_div(MI, 128); a.y = act; a.ldy = MI; a.MI = MI;
-  rc = launch_gemm<1>(a, mtiles_max, st);
-  if (rc) return rc;
-  rc = launch_rows_to_f16(act, R, MI, rmax, rexp_a, act16, nullptr, 0, st);
-  if (rc) return rc;
-  GemmArgs d = a;
-  d.a16 = act16; d.lda = MI; d.a_bytes = (uint32_t)((size_t)R * MI * 2); d.perm = (const int64_t*)order; d.topk = k; d.rexp = rexp_a; d.rmax_out = nullptr;
-  d.w = (const uint32_t*)dn_w; d.s = (const uint16_t*)dn_s; d.K = MI; d.N = H; d.gs = gs_dn;
-  d.n_ntiles = host_ceil_div(H, 256); d.y = prod; d.ldy = H; d.wts = (const uint16_t*)wts;
-  rc = launch_gemm<2>(d, mtiles_max, st);
-  if (rc) return rc;
+  int rc;
+  if (tile_rows_max != BM) {
+    FewRowsArgs f{};
+    f.x = (const uint16_t*)x; f.perm = (const int64_t*)order; f.topk = k;
+    f.w = (const uint32_t*)gu_w; f.s = (const uint16_t*)gu_s; f.K = H; f.N = 2 * MI; f.gs = gs_gu;
+    f.tile_expert = (const int*)tile_expert; f.tile_row0 = (const int*)tile_row0;
+    f.tile_rows = (const int*)tile_rows; f.tile_count = (const int*)tile_count; f.mtiles_max = mtiles_max;
+    f.R = R; f.y = act; f.ldy = MI; f.MI = MI;
+    rc = launch_w4_few_rows(1, f, st);
+    if (rc) return rc;
+    f.x = act; f.w = (const uint32_t*)dn_w; f.s = (const uint16_t*)dn_s; f.K = MI; f.N = H; f.gs = gs_dn;
+    f.y = prod; f.ldy = H; f.wts = (const uint16_t*)wts;
+    rc = launch_w4_few_rows(2, f, st);
+    if (rc) return rc;
+  } else {
+    rc = launch_rows_to_f16(x, T, H, nullptr, rexp_x, x16, rmax, R, st);
+    if (rc) return rc;
+    GemmArgs a{};
+    a.a16 = x16; a.lda = H; a.a_bytes = (uint32_t)((size_t)T * H * 2); a.perm = (const int64_t*)order; a.topk = k; a.rexp = rexp_x; a.rmax_out = rmax;
+    a.w = (const uint32_t*)gu_w; a.s = (const uint16_t*)gu_s; a.K = H; a.N = 2 * MI; a.gs = gs_gu;
+    a.tile_expert = (const int*)tile_expert; a.tile_row0 = (const int*)tile_row0;
+    a.tile_rows = (const int*)tile_rows; a.tile_count = (const int*)tile_count; a.R = R;
+    a.n_ntiles = host_ceil_div(MI, 128); a.y = act; a.ldy = MI; a.MI = MI;
+    rc = launch_gemm<1>(a, mtiles_max, st);
+    if (rc) return rc;
+    rc = launch_rows_to_f16(act, R, MI, rmax, rexp_a, act16, nullptr, 0, st);
+    if (rc) return rc;
+    GemmArgs d = a;
+    d.a16 = act16; d.lda = MI; d.a_bytes = (uint32_t)((size_t)R * MI * 2); d.perm = (const int64_t*)order; d.topk = k; d.rexp = rexp_a; d.rmax_out = nullptr;
+    d.w = (const uint32_t*)dn_w; d.s = (const uint16_t*)dn_s; d.K = MI; d.N = H; d.gs = gs_dn;
+    d.n_ntiles = host_ceil_div(H, 256); d.y = prod; d.ldy = H; d.wts = (const uint16_t*)wts;
+    rc = launch_gemm<2>(d, mtiles_max, st);
+    if (rc) return rc;
+  }
   // one workgroup row covers a token's H / 8 column groups (whole waves, at most 1024 threads), so no
   // thread of a launched block idles when H / 8 is a multiple of 64
   const int sr_threads = min(1024, host_ceil_div(H / 8, 64) * 64);
   hipLaunchKernelGGL(slot_reduce_kernel, dim3(host_ceil_div(H / 8, sr_threads), min(T, 65535)), dim3(sr_threads), 0, st, prod, T,
                      k, H, (const uint16_t*)shared, (uint16_t*)out);
   return (int)hipGetLastError();
+}
+
+int qmoe_moe_experts_grouped(const void* x, int T, int H, int MI, int E, int k, const void* wts,
+                             const void* order, const void* gu_w, const void* gu_s, int gs_gu,
+                             const void* dn_w, const void* dn_s, int gs_dn, const void* tile_expert,
+                             const void* tile_row0, const void* tile_rows, const void* tile_count,
+                             int mtiles_max, const void* shared, void* out, void* workspace,
+                             size_t workspace_bytes, void* stream) {
+  return qmoe_moe_experts_grouped_rows(x, T, H, MI, E, k, wts, order, gu_w, gu_s, gs_gu, dn_w, dn_s, gs_dn, BM,
+                                       tile_expert, tile_row0, tile_rows, tile_count, mtiles_max, shared, out,
+                                       workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

@@ -294,6 +294,41 @@ QMOE_DEV void wave_topk_softmax(const uint16_t* __restrict__ logits, int E, int 
   wave_route_softmax<KPL>(lg, E, k, sel, idx_out, w_out);
 }
 
+// ---------------------------------------------------------------- MFMA kernels: waits, conversions
+
+typedef float f32x2_v __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
+
+// s_waitcnt with vmcnt <= N and lgkmcnt == 0 (gfx9 encoding: vmcnt bits
+// [3:0] and [15:14], expcnt [6:4] left at 7).
+template <int N>
+QMOE_DEV void wait_vm_lgkm0() {
+  static_assert(N >= 0 && N < 64, "vmcnt range");
+  __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4));
+}
+
+// Workgroup barrier without a memory fence: the caller has already waited
+// for the memory operations the barrier must order (a fence here would also
+// wait for the prefetches still in flight).
+QMOE_DEV void barrier_no_fence() {
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+QMOE_DEV uint32_t pk_rtz(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(lo, hi));
+}
+// bf16 pair (RNE, hardware conversion; finite values round exactly like f32_to_bf16)
+QMOE_DEV uint32_t pk_bf16(float lo, float hi) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2_v){lo, hi}, bf16x2_v));
+}
+
+// exponent that brings a magnitude with bf16 biased exponent eb into [2^t, 2^(t+1)), t = target - 127
+QMOE_DEV int exp_to(uint32_t max_abs_bits, int target_biased) {
+  const int eb = (int)(max_abs_bits >> 7) & 0xff;
+  return eb == 0 ? 0 : target_biased - eb;
+}
+
 // ---------------------------------------------------------------- cross-workgroup hand-off
 //
 // Partial results that another workgroup of the same launch reduces are

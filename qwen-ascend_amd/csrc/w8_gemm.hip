@@ -156,14 +156,6 @@ QMOE_DEV uint32_t i8_to_bf16_bits(uint32_t word, int byte) {
   return __float_as_uint((float)(int)(int8_t)(word >> (8 * byte))) >> 16;
 }
 
-// s_waitcnt with vmcnt <= N and lgkmcnt == 0 (gfx9 encoding: vmcnt bits
-// [3:0] and [15:14], expcnt [6:4] left at 7).
-template <int N>
-QMOE_DEV void wait_vm_lgkm0() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4));
-}
-
 // An 8-byte LDS write the compiler does not track. It cannot tell which LDS
 // bytes an in-flight global->LDS DMA writes, so before an ordinary LDS store
 // it would wait for every outstanding DMA (the chunks prefetched ahead too);

@@ -54,11 +54,15 @@ SIGNATURES = {
     "qmoe_tiles_from_ends": (I, [P, I, I, I, P, P, P, P, P]),
     "qmoe_tiles_from_ids": (I, [P, I, I, P, P, P, P, P]),
     "qmoe_gemm_tile_rows": (I, []),
+    "qmoe_gemm_tile_rows_for": (I, [I, I, I, I, I]),
+    "qmoe_moe_tile_rows": (I, [I, I, I, I, I, I]),
     "qmoe_grouped_gemm_workspace": (Z, [I, I]),
     "qmoe_grouped_gemm": (I, [P, I, I, I, I, I, P, P, P, P, P, P, I, P, P, Z, P]),
+    "qmoe_grouped_gemm_rows": (I, [P, I, I, I, I, I, P, P, I, P, P, P, P, I, P, P, Z, P]),
     "qmoe_moe_prefill_workspace": (Z, [I, I, I, I]),
     "qmoe_moe_prefill_layout": (I, [I, I, I, I, P, P]),
     "qmoe_moe_experts_grouped": (I, [P, I, I, I, I, I, P, P, P, P, I, P, P, I, P, P, P, P, I, P, P, P, Z, P]),
+    "qmoe_moe_experts_grouped_rows": (I, [P, I, I, I, I, I, P, P, P, P, I, P, P, I, I, P, P, P, P, I, P, P, P, Z, P]),
     "qmoe_expert_gather": (I, [P, P, P, P, P, I, I, I, I, I, P]),
     "qmoe_expert_gather_kmajor": (I, [P, P, P, P, P, I, I, I, I, I, P]),
     "qmoe_weighted_reduce": (I, [P, P, P, P, I, I, I, L, L, P]),

@@ -207,10 +207,11 @@ class ExpW4:
                                          tcnt.data_ptr(), st), "apply_diag tiles")
         y = torch.empty((k, self.N), dtype=BF16, device=dev)
         ws = _lib.workspace(dev, L.qmoe_grouped_gemm_workspace(k, self.K))
-        _lib.check(L.qmoe_grouped_gemm(x.data_ptr(), k, self.K, self.N, self.E, self.gs, self.w4.data_ptr(),
-                                       self._scales.data_ptr(), te.data_ptr(), tr0.data_ptr(), trows.data_ptr(),
-                                       tcnt.data_ptr(), k, y.data_ptr(), ws.data_ptr(), ws.numel(), st),
-                   "apply_diag")
+        bm = L.qmoe_gemm_tile_rows_for(k, self.E, self.K, self.N, self.gs)
+        _lib.check(L.qmoe_grouped_gemm_rows(x.data_ptr(), k, self.K, self.N, self.E, self.gs, self.w4.data_ptr(),
+                                            self._scales.data_ptr(), bm, te.data_ptr(), tr0.data_ptr(),
+                                            trows.data_ptr(), tcnt.data_ptr(), k, y.data_ptr(), ws.data_ptr(),
+                                            ws.numel(), st), "apply_diag")
         return y
 
     def apply_grouped(self, x, group_ends, host_ends=None):
@@ -407,14 +408,15 @@ def moe_prefill(x, logits, exp_gu, exp_dn, topk, shared=None, return_routing=Fal
     MI = exp_dn.K
     E = exp_gu.E
     idx, w = router_topk(logits, topk)
-    counts, ends, order, inverse, tiles, mt = route_group(idx, E, with_tiles=True)
-    out = torch.empty((T, H), dtype=BF16, device=dev)
     L = _lib.lib()
+    bm = L.qmoe_moe_tile_rows(T * topk, E, H, MI, exp_gu.gs, exp_dn.gs)
+    counts, ends, order, inverse, tiles, mt = route_group(idx, E, with_tiles=True, tile_rows=bm)
+    out = torch.empty((T, H), dtype=BF16, device=dev)
     ws = _lib.workspace(dev, L.qmoe_moe_prefill_workspace(T, topk, H, MI))
     sh = shared.contiguous() if shared is not None else None
-    rc = L.qmoe_moe_experts_grouped(
+    rc = L.qmoe_moe_experts_grouped_rows(
         x.data_ptr(), T, H, MI, E, topk, w.data_ptr(), order.data_ptr(), exp_gu.w4.data_ptr(),
-        exp_gu._scales.data_ptr(), exp_gu.gs, exp_dn.w4.data_ptr(), exp_dn._scales.data_ptr(), exp_dn.gs,
+        exp_gu._scales.data_ptr(), exp_gu.gs, exp_dn.w4.data_ptr(), exp_dn._scales.data_ptr(), exp_dn.gs, bm,
         tiles[:mt].data_ptr(), tiles[mt:2 * mt].data_ptr(), tiles[2 * mt:3 * mt].data_ptr(),
         tiles[3 * mt:].data_ptr(), mt, _lib.ptr(sh), out.data_ptr(), ws.data_ptr(), ws.numel(),
         _lib.stream_of(x))

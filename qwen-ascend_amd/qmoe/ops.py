@@ -111,9 +111,9 @@ def _w8a16(x, weight, scale, gs):
     return y
 
 
-def _tile_table(R, E, device):
+def _tile_table(R, E, device, bm=None):
     L = _lib.lib()
-    bm = L.qmoe_gemm_tile_rows()
+    bm = L.qmoe_gemm_tile_rows() if bm is None else bm
     mt = L.qmoe_max_row_tiles(R, E, bm)
     tiles = torch.empty((3 * mt + 1,), dtype=torch.int32, device=device)
     return bm, mt, tiles
@@ -163,14 +163,14 @@ def grouped_matmul(x, weight, *, bias=None, scale=None, offset=None, antiquant_s
         return [y]
     L = _lib.lib()
     st = _lib.stream_of(xt)
-    bm, mt, tiles = _tile_table(R, E, xt.device)
+    bm, mt, tiles = _tile_table(R, E, xt.device, L.qmoe_gemm_tile_rows_for(R, E, K, N, gs))
     te, tr0, trows, tcount = tiles[:mt], tiles[mt:2 * mt], tiles[2 * mt:3 * mt], tiles[3 * mt:]
     _lib.check(L.qmoe_tiles_from_ends(gl.data_ptr(), E, R, bm, te.data_ptr(), tr0.data_ptr(),
                                       trows.data_ptr(), tcount.data_ptr(), st), "grouped_matmul tiles")
     ws = _lib.workspace(xt.device, L.qmoe_grouped_gemm_workspace(R, K))
-    _lib.check(L.qmoe_grouped_gemm(xt.data_ptr(), R, K, N, E, gs, w.data_ptr(), s.data_ptr(), te.data_ptr(),
-                                   tr0.data_ptr(), trows.data_ptr(), tcount.data_ptr(), mt, y.data_ptr(),
-                                   ws.data_ptr(), ws.numel(), st), "grouped_matmul")
+    _lib.check(L.qmoe_grouped_gemm_rows(xt.data_ptr(), R, K, N, E, gs, w.data_ptr(), s.data_ptr(), bm, te.data_ptr(),
+                                        tr0.data_ptr(), trows.data_ptr(), tcount.data_ptr(), mt, y.data_ptr(),
+                                        ws.data_ptr(), ws.numel(), st), "grouped_matmul")
     return [y]
 
 
@@ -209,13 +209,14 @@ def router_topk(logits, k):
     return idx, w
 
 
-def route_group(idx, E, with_tiles=False):
+def route_group(idx, E, with_tiles=False, tile_rows=None):
     """Expert-major grouping of routed ids (``fnx/engine.py:1816-1823, 1832-1843``).
 
     Returns (counts, ends, order, inverse) int64 — ends is the inclusive
     cumsum (``group_list``), order the stable expert-major permutation of the
     flat ids, inverse[order[p]] = p. With ``with_tiles`` also the grouped
-    GEMM row-tile table (tile tensor, max tiles).
+    GEMM row-tile table (tile tensor, max tiles) of tiles of at most
+    ``tile_rows`` rows (``qmoe_gemm_tile_rows()`` by default).
     """
     if idx.dtype != torch.int64:
         raise RuntimeError("ids must be int64")
@@ -228,7 +229,7 @@ def route_group(idx, E, with_tiles=False):
     order = torch.empty((R,), dtype=torch.int64, device=dev)
     inverse = torch.empty((R,), dtype=torch.int64, device=dev)
     L = _lib.lib()
-    bm, mt, tiles = _tile_table(R, E, dev)
+    bm, mt, tiles = _tile_table(R, E, dev, tile_rows)
     ws = _lib.workspace(dev, L.qmoe_route_group_workspace(R, E))
     te, tr0, trows, tcount = tiles[:mt], tiles[mt:2 * mt], tiles[2 * mt:3 * mt], tiles[3 * mt:]
     _lib.check(L.qmoe_route_group(ids.data_ptr(), R, E, counts.data_ptr(), ends.data_ptr(), order.data_ptr(),
