@@ -330,6 +330,12 @@ int qmoe_bf16_gemv_split(const void* x, long ldx, const void* w, void* y, long l
  * GEMM): K % 32 == 0, ldx % 8 == 0, x and w 16-byte aligned, any M and N
  * with x's and w's extents ((M-1)*ldx + K and N*K elements) under 2^30. */
 int qmoe_bf16_gemm(const void* x, long ldx, const void* w, void* y, long ldy, int M, int K, int N, void* stream);
+/* The same for the fused shared-expert projection W = [gate MI | up MI | rest]
+ * (fnx/engine.py:1226-1241, 1787-1788): columns [2 MI, N) go to y (at their
+ * place; the first 2 MI columns of y are not written), and act bf16 [M, MI] =
+ * bf16(bf16(silu(g)) * u) of the first 2 MI columns' bf16 values. N > 2 MI. */
+int qmoe_bf16_gemm_swiglu(const void* x, long ldx, const void* w, void* y, long ldy, void* act, int M, int K, int N,
+                          int MI, void* stream);
 /* The same with the shared expert's SwiGLU as the activations, read from the
  * first projection gu: a[m,k] = bf16(bf16(silu(gu[m,k])) * gu[m,MI+k])
  * (F.silu(gu[:, :MI]) * gu[:, MI:2MI], fnx/engine.py:1788); K = MI. */

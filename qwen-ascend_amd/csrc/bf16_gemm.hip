@@ -13,7 +13,10 @@
 // RING LDS slots by buffer-resource global->LDS DMA, RING - 1 chunks ahead,
 // the 16-byte pieces of every row stored XOR-swizzled by row so the 16 rows a
 // fragment read touches fall in different banks. One barrier per chunk.
-// Workgroups that share rows of a run on one XCD. Products of two bf16 are
+// Workgroups that share rows of a run on one XCD. Outputs of a few tiles take a
+// kernel of their own (below). SWIGLU (the fused shared-expert projection, W =
+// [gate MI | up MI | rest]): the first 2 MI columns leave as the SwiGLU rows
+// act = bf16(bf16(silu(g)) * u) of their bf16 results instead of y. Products of two bf16 are
 // exact in fp32, so the result is the rounding of an fp32 accumulation of
 // exact terms.
 #include "qmoe_common.h"
@@ -43,18 +46,29 @@ struct Bf16Tile {
   static_assert(A_BYTES % 4096 == 0 && B_BYTES % 4096 == 0, "tile shape");
 };
 
-template <class T>
+template <class T, bool SWIGLU>
 __global__ __launch_bounds__(kThreads) void bf16_gemm_kernel(const uint16_t* __restrict__ a, long lda,
                                                              const uint16_t* __restrict__ w, uint16_t* __restrict__ y,
-                                                             long ldy, int M, int K, int N) {
+                                                             long ldy, int M, int K, int N, uint16_t* __restrict__ act,
+                                                             int MI) {
   constexpr int BM = T::BM, BN = T::BN, KC = T::KC, RING = T::RING;
   constexpr int TI = T::TI, TJ = T::TJ, PPR = T::PPR;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int ntn = (N + BN - 1) / BN;
+  const int act_tiles = SWIGLU ? (MI + BN / 2 - 1) / (BN / 2) : 0;
+  const int ntn = act_tiles + (N - (SWIGLU ? 2 * MI : 0) + BN - 1) / BN;
   const int ntiles = ((M + BM - 1) / BM) * ntn;
   const int tile = xcd_remap(blockIdx.x, gridDim.x);
   if (tile >= ntiles) return;
-  const int m0 = (tile / ntn) * BM, n0 = (tile % ntn) * BN;
+  const int m0 = (tile / ntn) * BM, nt = tile % ntn;
+  const bool sw = SWIGLU && nt < act_tiles;
+  const int n0 = SWIGLU && !sw ? 2 * MI + (nt - act_tiles) * BN : nt * BN;
+  // tile column c -> row of w (rows past the last re-read it, never stored). A
+  // SwiGLU tile: columns c with c / 16 even are gate rows, odd the up rows of
+  // the same act columns, so a lane holds both of an act column.
+  auto wrow = [&](int c) {
+    if (sw) return ((c >> 4) & 1) * MI + min(nt * (BN / 2) + 16 * (c >> 5) + (c & 15), MI - 1);
+    return min(n0 + c, N - 1);
+  };
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int wm = wave >> 1, wn = wave & 1;
@@ -79,7 +93,7 @@ __global__ __launch_bounds__(kThreads) void bf16_gemm_kernel(const uint16_t* __r
 #pragma unroll
   for (int q = 0; q < T::BQ; ++q) {
     const int r = (64 / PPR) * (4 * q + wave) + lane / PPR;
-    boff[q] = 2u * ((uint32_t)min(n0 + r, N - 1) * (uint32_t)K + 8u * (uint32_t)((lane % PPR) ^ swz(r)));
+    boff[q] = 2u * ((uint32_t)wrow(r) * (uint32_t)K + 8u * (uint32_t)((lane % PPR) ^ swz(r)));
   }
   auto issue_chunk = [&](int c) {
     unsigned char* base = lds + (c % RING) * T::SLOT;
@@ -142,6 +156,21 @@ __global__ __launch_bounds__(kThreads) void bf16_gemm_kernel(const uint16_t* __r
   }
 
   // lane holds column i16 of tile (i, j) for rows 4*kb + r
+  if (sw) {
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; j += 2) {
+        const int n = nt * (BN / 2) + 16 * ((wn * (BN / 2) + 16 * j) >> 5) + i16;
+        if (n >= MI) continue;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + wm * (BM / 2) + i * 16 + 4 * kb + r;
+          if (m < M) act[(size_t)m * MI + n] = (uint16_t)swiglu_bf16_bits(f32_to_bf16(acc[i][j][r]), f32_to_bf16(acc[i][j + 1][r]));
+        }
+      }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -156,25 +185,227 @@ __global__ __launch_bounds__(kThreads) void bf16_gemm_kernel(const uint16_t* __r
     }
 }
 
-template <class T>
-int launch_bf16_gemm(const void* x, long ldx, const void* w, void* y, long ldy, int M, int K, int N,
-                     hipStream_t stream) {
+struct Bf16Args {
+  const uint16_t* x;
+  long ldx;
+  const uint16_t* w;
+  uint16_t* y;
+  long ldy;
+  int M, K, N;
+  uint16_t* act;  // SwiGLU form: act rows of the first 2 MI columns
+  int MI;
+};
+
+template <bool SWIGLU>
+long col_tiles(const Bf16Args& a, int bn) {
+  return SWIGLU ? (long)host_ceil_div(a.MI, bn / 2) + host_ceil_div(a.N - 2 * a.MI, bn) : host_ceil_div(a.N, bn);
+}
+
+template <class T, bool SWIGLU>
+int launch_bf16_gemm(const Bf16Args& a, hipStream_t stream) {
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return (int)err;
   if (dev < 0 || dev >= 64) return QMOE_EINVAL;
   static bool attr_set[64] = {};
   if (!attr_set[dev]) {
-    err = hipFuncSetAttribute((const void*)bf16_gemm_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+    err = hipFuncSetAttribute((const void*)bf16_gemm_kernel<T, SWIGLU>, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
     if (err != hipSuccess) return (int)err;
     attr_set[dev] = true;
   }
-  const long tiles = (long)((M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN);
+  const long tiles = (long)host_ceil_div(a.M, T::BM) * col_tiles<SWIGLU>(a, T::BN);
   const long blocks = (tiles + 7) / 8 * 8;  // whole XCD rounds (extra blocks exit)
   if (blocks > 0x7fffffffL) return QMOE_EINVAL;
-  hipLaunchKernelGGL(bf16_gemm_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), T::LDS, stream, (const uint16_t*)x,
-                     ldx, (const uint16_t*)w, (uint16_t*)y, ldy, M, K, N);
+  hipLaunchKernelGGL((bf16_gemm_kernel<T, SWIGLU>), dim3((unsigned)blocks), dim3(kThreads), T::LDS, stream, a.x, a.ldx, a.w,
+                     a.y, a.ldy, a.M, a.K, a.N, a.act, a.MI);
   return (int)hipGetLastError();
+}
+
+// ---------------------------------------------------------------- few tiles: K split over the waves
+//
+// 16 LIVE rows of a times 16 F columns per workgroup; the NW waves split K
+// (contiguous runs of 32-k steps) and load both operands' fragments straight
+// into registers (a fragment is one 16-byte piece per lane), U steps as one
+// batch while the previous batch's MFMAs run. The waves' partial tiles meet in
+// LDS and are summed in wave order: the same bits every run. SWIGLU: the tiles of
+// the first 2 MI columns take 8 F gate columns, then their 8 F up columns.
+//
+// What bounds it: launch and first load (about 4 us) and the (LIVE + F) KB per
+// step that a CU draws from L2 at some 27 bytes per clock. 2560 x 1793: 7.2 us
+// at 5 rows (1.3 TB/s of cold weights) and 11.3 at 64, against 19.4 and 24.1 of
+// the 64 x 64 LDS-ring tile, whose one chain of 32-k chunks ran on 29 CUs;
+// 2048 x 512 at 200 rows 7.9 against 14.4.
+template <int LIVE, int F, int NW, int U, bool SWIGLU>
+__global__ __launch_bounds__(64 * NW) void bf16_skinny_kernel(Bf16Args g) {
+  constexpr int BN = 16 * F, ROWS = 16 * LIVE, LDR = BN + 4;  // LDS row: the four k-blocks' rows in different banks
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  float* red = reinterpret_cast<float*>(lds);  // [NW][ROWS][LDR]
+  const int M = g.M, K = g.K, N = g.N, MI = g.MI;
+  const int nrg = (M + ROWS - 1) / ROWS;
+  const int act_tiles = SWIGLU ? (MI + BN / 2 - 1) / (BN / 2) : 0;
+  const int ntn = act_tiles + (N - (SWIGLU ? 2 * MI : 0) + BN - 1) / BN;
+  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  if (tile >= nrg * ntn) return;
+  const int m0 = (tile % nrg) * ROWS, nt = tile / nrg;
+  const bool sw = SWIGLU && nt < act_tiles;
+  const int n0 = SWIGLU && !sw ? 2 * MI + (nt - act_tiles) * BN : nt * BN;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i16 = lane & 15, kb = lane >> 4;
+  // tile column c -> row of w (rows past the last re-read it, never stored)
+  auto wrow = [&](int c) {
+    if (sw) return (c / (BN / 2)) * MI + min(nt * (BN / 2) + c % (BN / 2), MI - 1);
+    return min(n0 + c, N - 1);
+  };
+  constexpr int kRsrcWord3 = 0x00020000;
+  const __amdgpu_buffer_rsrc_t rsrc_a =
+      __builtin_amdgcn_make_buffer_rsrc((void*)g.x, (short)0, (int)(((long)(M - 1) * g.ldx + K) * 2), kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)g.w, (short)0, N * K * 2, kRsrcWord3);
+  int aoff[LIVE], boff[F];
+#pragma unroll
+  for (int t = 0; t < LIVE; ++t) aoff[t] = (int)(2 * ((long)min(m0 + 16 * t + i16, M - 1) * g.ldx + 8 * kb));
+#pragma unroll
+  for (int f = 0; f < F; ++f) boff[f] = 2 * (wrow(16 * f + i16) * K + 8 * kb);
+  const int nsteps = K / BK, per = (nsteps + NW - 1) / NW;
+  const int s0 = min(nsteps, wave * per), s1 = min(nsteps, s0 + per);
+  f32x4_v acc[LIVE][F];
+#pragma unroll
+  for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+    for (int f = 0; f < F; ++f) acc[t][f] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+  struct Batch {
+    bf16x8_v a[U][LIVE], b[U][F];
+  };
+  auto load = [&](int st, Batch& v) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int off = 2 * BK * min(st + u, s1 - 1);  // past the run's end its last step (not used)
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+        v.b[u][f] = __builtin_bit_cast(bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(rsrc_b, boff[f], off, 0));
+#pragma unroll
+      for (int t = 0; t < LIVE; ++t)
+        v.a[u][t] = __builtin_bit_cast(bf16x8_v, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, aoff[t], off, 0));
+    }
+  };
+  auto mma = [&](int st, const Batch& v) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (st + u >= s1) break;
+#pragma unroll
+      for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+          acc[t][f] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v.a[u][t], v.b[u][f], acc[t][f], 0, 0, 0);
+    }
+  };
+  if (s0 < s1) {
+    Batch v0, v1;
+    load(s0, v0);
+    for (int st = s0; st < s1; st += 2 * U) {
+      if (st + U < s1) load(st + U, v1);
+      mma(st, v0);
+      if (st + 2 * U < s1) load(st + 2 * U, v0);
+      if (st + U < s1) mma(st + U, v1);
+    }
+  }
+  // lane holds column i16 of each fragment for rows 4 kb + r
+#pragma unroll
+  for (int t = 0; t < LIVE; ++t)
+#pragma unroll
+    for (int f = 0; f < F; ++f)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[((size_t)wave * ROWS + 16 * t + 4 * kb + r) * LDR + 16 * f + i16] = acc[t][f][r];
+  __syncthreads();
+  auto total = [&](int row, int c) {
+    float v = red[row * LDR + c];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) v += red[((size_t)q * ROWS + row) * LDR + c];
+    return v;
+  };
+  const int rows = min(ROWS, M - m0);
+  if (sw) {
+    for (int p = tid; p < rows * (BN / 2); p += 64 * NW) {
+      const int row = p / (BN / 2), c = p % (BN / 2), col = nt * (BN / 2) + c;
+      const uint32_t gb = f32_to_bf16(total(row, c)), ub = f32_to_bf16(total(row, BN / 2 + c));
+      if (col < MI) g.act[(size_t)(m0 + row) * MI + col] = (uint16_t)swiglu_bf16_bits(gb, ub);
+    }
+    return;
+  }
+  for (int p = tid; p < rows * BN; p += 64 * NW) {
+    const int row = p / BN, c = p % BN;
+    if (n0 + c < N) g.y[(size_t)(m0 + row) * g.ldy + n0 + c] = (uint16_t)f32_to_bf16(total(row, c));
+  }
+}
+
+template <int LIVE, int F, int NW, int U, bool SWIGLU>
+int launch_bf16_skinny(const Bf16Args& a, hipStream_t stream) {
+  constexpr int kLds = NW * 16 * LIVE * (16 * F + 4) * 4;
+  static_assert(kLds <= 160 * 1024, "LDS of a CU");
+  int dev = 0;
+  hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return (int)err;
+  if (dev < 0 || dev >= 64) return QMOE_EINVAL;
+  static bool attr_set[64] = {};
+  auto* kern = bf16_skinny_kernel<LIVE, F, NW, U, SWIGLU>;
+  if (!attr_set[dev]) {
+    err = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    if (err != hipSuccess) return (int)err;
+    attr_set[dev] = true;
+  }
+  const long blocks = (host_ceil_div(a.M, 16 * LIVE) * col_tiles<SWIGLU>(a, 16 * F) + 7) / 8 * 8;  // whole XCD rounds
+  if (blocks > 0x7fffffffL) return QMOE_EINVAL;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(64 * NW), kLds, stream, a);
+  return (int)hipGetLastError();
+}
+
+// The skinny kernel where a tile of at most four fragments (LIVE + F) covers
+// the output in one round of the 256 CUs; false where none does.
+// Eight waves with longer batches for a long K (2560 x 1793 at 48 rows 11.0
+// against 11.5 us with 16), 16 for a short one (640 x 2560 4.4 against 5.0).
+template <bool SWIGLU>
+bool launch_bf16_few_tiles(const Bf16Args& a, hipStream_t st, int* rc) {
+  auto fits = [&](int live, int f) { return host_ceil_div(a.M, 16 * live) * col_tiles<SWIGLU>(a, 16 * f) <= 256; };
+  const bool long_k = a.K >= 1536;
+#define QMOE_SKINNY(L_, F_, U8_, U16_)                                                 \
+  if (fits(L_, F_)) {                                                                  \
+    *rc = long_k ? launch_bf16_skinny<L_, F_, 8, U8_, SWIGLU>(a, st)                   \
+                 : launch_bf16_skinny<L_, F_, 16, U16_, SWIGLU>(a, st);                \
+    return true;                                                                       \
+  }
+  QMOE_SKINNY(1, 1, 4, 2) QMOE_SKINNY(1, 2, 4, 2) QMOE_SKINNY(2, 1, 4, 2) QMOE_SKINNY(2, 2, 2, 2)
+  QMOE_SKINNY(3, 1, 2, 2)
+#undef QMOE_SKINNY
+  return false;
+}
+
+template <bool SWIGLU>
+int run_bf16_gemm(const Bf16Args& a, hipStream_t st) {
+  int rc = QMOE_OK;
+  if (launch_bf16_few_tiles<SWIGLU>(a, st, &rc)) return rc;
+  // 64 x 64 tiles while each has a CU of its own: 128-k chunks in three slots
+  // (2560 x 1793 at 200 rows 13.7 us against 20.3 with 32-k chunks in four, 14.3
+  // with 64-k ones; K split over two rings per workgroup: no gain, 13.5).
+  if ((long)host_ceil_div(a.M, 64) * col_tiles<SWIGLU>(a, 64) <= 256) {
+    if (a.K % 128 == 0) return launch_bf16_gemm<Bf16Tile<64, 64, 128, 3>, SWIGLU>(a, st);
+    if (a.K % 64 == 0) return launch_bf16_gemm<Bf16Tile<64, 64, 64, 4>, SWIGLU>(a, st);
+    return launch_bf16_gemm<Bf16Tile<64, 64, 32, 4>, SWIGLU>(a, st);
+  }
+  // 128 x 128 tiles where they give every CU two workgroups, else 128 x 64
+  // (3072 x 2049 at 512 rows 25.2 us against 33.4 with 64 x 64). 64-k chunks,
+  // double-buffered at 128 x 128, where K allows (4096 x 3072 x 2048: 650 -> 980
+  // TFLOP/s against 32-k chunks in a 4-slot ring: half the barriers and waits
+  // per MFMA)
+  if ((long)host_ceil_div(a.M, 128) * col_tiles<SWIGLU>(a, 128) >= 512)
+    return a.K % 64 == 0 ? launch_bf16_gemm<Bf16Tile<128, 128, 64, 2>, SWIGLU>(a, st)
+                         : launch_bf16_gemm<Bf16Tile<128, 128, 32, 4>, SWIGLU>(a, st);
+  return a.K % 64 == 0 ? launch_bf16_gemm<Bf16Tile<128, 64, 64, 3>, SWIGLU>(a, st)
+                       : launch_bf16_gemm<Bf16Tile<128, 64, 32, 4>, SWIGLU>(a, st);
+}
+
+bool bf16_gemm_ok(const void* x, long ldx, const void* w, long ldy, int M, int K, int N) {
+  return M >= 1 && N >= 1 && K >= BK && K % BK == 0 && ldx >= K && ldx % 8 == 0 && ldy >= N && ((uintptr_t)x & 15) == 0 &&
+         ((uintptr_t)w & 15) == 0 && ((long)(M - 1) * ldx + K) * 2 < 0x80000000L && (long)N * K * 2 < 0x80000000L;
 }
 
 }  // namespace
@@ -182,24 +413,16 @@ int launch_bf16_gemm(const void* x, long ldx, const void* w, void* y, long ldy, 
 extern "C" {
 
 int qmoe_bf16_gemm(const void* x, long ldx, const void* w, void* y, long ldy, int M, int K, int N, void* stream) {
-  if (M < 1 || N < 1 || K < BK || (K % BK) || ldx < K || (ldx % 8) || ldy < N ||
-      ((uintptr_t)x & 15) || ((uintptr_t)w & 15) ||
-      ((long)(M - 1) * ldx + K) * 2 >= 0x80000000L || (long)N * K * 2 >= 0x80000000L)
-    return QMOE_EINVAL;
-  hipStream_t st = (hipStream_t)stream;
-  // 128 x 128 tiles where they give every CU two workgroups, else 128 x 64
-  // (64-k chunks when K allows) where they give every CU one, else 64 x 64
-  const long tiles128 = (long)((M + 127) / 128) * ((N + 63) / 64);
-  const long tiles128x128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-  // 64-k chunks double-buffered where K allows (4096 x 3072 x 2048: 650 -> 980
-  // TFLOP/s against 32-k chunks in a 4-slot ring: half the barriers and waits
-  // per MFMA)
-  if (tiles128x128 >= 512 && K % 64 == 0)
-    return launch_bf16_gemm<Bf16Tile<128, 128, 64, 2>>(x, ldx, w, y, ldy, M, K, N, st);
-  if (tiles128x128 >= 512) return launch_bf16_gemm<Bf16Tile<128, 128, 32, 4>>(x, ldx, w, y, ldy, M, K, N, st);
-  if (tiles128 >= 256 && K % 64 == 0) return launch_bf16_gemm<Bf16Tile<128, 64, 64, 3>>(x, ldx, w, y, ldy, M, K, N, st);
-  if (tiles128 >= 256) return launch_bf16_gemm<Bf16Tile<128, 64, 32, 4>>(x, ldx, w, y, ldy, M, K, N, st);
-  return launch_bf16_gemm<Bf16Tile<64, 64, 32, 4>>(x, ldx, w, y, ldy, M, K, N, st);
+  if (!bf16_gemm_ok(x, ldx, w, ldy, M, K, N)) return QMOE_EINVAL;
+  return run_bf16_gemm<false>({(const uint16_t*)x, ldx, (const uint16_t*)w, (uint16_t*)y, ldy, M, K, N, nullptr, 0},
+                              (hipStream_t)stream);
+}
+
+int qmoe_bf16_gemm_swiglu(const void* x, long ldx, const void* w, void* y, long ldy, void* act, int M, int K, int N,
+                          int MI, void* stream) {
+  if (!bf16_gemm_ok(x, ldx, w, ldy, M, K, N) || MI < 1 || N <= 2 * MI) return QMOE_EINVAL;
+  return run_bf16_gemm<true>({(const uint16_t*)x, ldx, (const uint16_t*)w, (uint16_t*)y, ldy, M, K, N, (uint16_t*)act, MI},
+                             (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -75,6 +75,7 @@ SIGNATURES = {
     "qmoe_bf16_gemv": (I, [P, L, P, P, L, I, I, I, P]),
     "qmoe_bf16_gemv_split": (I, [P, L, P, P, L, P, L, I, I, I, I, P]),
     "qmoe_bf16_gemm": (I, [P, L, P, P, L, I, I, I, P]),
+    "qmoe_bf16_gemm_swiglu": (I, [P, L, P, P, L, P, I, I, I, I, P]),
     "qmoe_bf16_gemv_swiglu": (I, [P, L, P, P, L, I, I, I, P]),
     "qmoe_swiglu_bf16": (I, [P, L, P, L, I, P]),
     "qmoe_shared_gate": (I, [P, P, L, P, L, I, P]),

@@ -10,8 +10,8 @@ weight, ``fnx/engine.py:1226-1241``):
 
 One to four rows run the hand-written bf16 GEMVs of libqmoe.so (the shared
 SwiGLU is computed inside the second one); larger batches run the two
-projections on the hand-written bf16 MFMA GEMM with the SwiGLU and gate
-kernels of libqmoe.so. :func:`moe_block` chains this with the expert block: at decode
+projections on the hand-written bf16 MFMA GEMM, the first one's epilogue
+computing the SwiGLU, and the gate kernel of libqmoe.so. :func:`moe_block` chains this with the expert block: at decode
 the sigmoid-gated shared merge is fused into the experts' epilogue
 (``fnx/engine.py:1790-1791, 1884-1891``); for larger batches the shared
 output is gated first, ``sh = sigmoid(gate2) * sh`` (``fnx/engine.py:1793``),
@@ -49,8 +49,10 @@ def linear(x, w):
     return _gemv(x, w, N)
 
 
-def _gemm(x, w, ldy=None):
-    """HIP MFMA GEMM into rows ldy >= N apart; returns the [M, N] view.
+def _gemm(x, w, ldy=None, MI=None):
+    """HIP MFMA GEMM into rows ldy >= N apart; returns the [M, N] view, or with
+    ``MI`` that view (its first 2 MI columns unwritten) and the SwiGLU rows
+    [M, MI] of those columns.
 
     The kernel reads 16-byte pieces of 32-wide K chunks: operands that start
     off a 16-byte boundary are copied to fresh (aligned) tensors, and a K that
@@ -72,6 +74,12 @@ def _gemm(x, w, ldy=None):
     if w.data_ptr() % 16:
         w = w.clone()
     y = torch.empty((M, ldy), dtype=BF16, device=x.device)
+    if MI is not None:
+        act = torch.empty((M, MI), dtype=BF16, device=x.device)
+        _lib.check(_lib.lib().qmoe_bf16_gemm_swiglu(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), ldy,
+                                                    act.data_ptr(), M, K, N, MI, _lib.stream_of(x)),
+                   "shared/router projection")
+        return y[:, :N], act
     _lib.check(_lib.lib().qmoe_bf16_gemm(x.data_ptr(), x.stride(0), w.data_ptr(), y.data_ptr(), ldy, M, K, N,
                                          _lib.stream_of(x)), "bf16 GEMM")
     return y[:, :N]
@@ -165,9 +173,8 @@ def shared_router(x2, sh_gu, sh_down, MI):
     b, H = x2.shape
     N, split = sh_gu.shape[0], 2 * MI + 1
     if b > DECODE_MAX_TOKENS:
-        gu = _gemm(x2, sh_gu, (N + 7) // 8 * 8)
-        sh = linear(swiglu_bf16(gu, MI), sh_down)
-        return sh, gu[:, 2 * MI:split], gu[:, split:]
+        gu, act = _gemm(x2, sh_gu, (N + 7) // 8 * 8, MI)
+        return linear(act, sh_down), gu[:, 2 * MI:split], gu[:, split:]
     gu, logits = _project(x2, sh_gu, MI)
     return _shared_down(gu, sh_down, MI, H), gu[:, 2 * MI:split], logits
 

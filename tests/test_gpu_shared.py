@@ -220,3 +220,26 @@ def test_moe_block_one_token_misaligned_falls_back(device):
     torch.cuda.synchronize()
     assert torch.equal(a.view(torch.int16), b.view(torch.int16))
     assert _lib.decode_status(_lib.counters(device)) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 17, 49, 300, 1100])
+@pytest.mark.parametrize("K,MI,rest", [(32, 8, 1), (64, 40, 9), (1536, 100, 300), (256, 1024, 513)])
+def test_bf16_gemm_swiglu(device, M, K, MI, rest):
+    """The fused projection's SwiGLU epilogue over its tile forms (ragged act
+    and rest columns). The operands are whole numbers whose sums are exact in
+    fp32 in any order, so every output bit is determined."""
+    from qmoe.shared import _gemm
+    log(f"bf16 GEMM swiglu M={M} K={K} MI={MI} rest={rest}")
+    r = np.random.default_rng(M + K)
+    x = r.integers(-3, 4, size=(M, K)).astype(np.float32)
+    w = r.integers(-2, 3, size=(2 * MI + rest, K)).astype(np.float32) / 16
+    gu = O.f32_to_bf16_bits((x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.float32))
+    N = 2 * MI + rest
+    y, act = _gemm(to_dev(O.f32_to_bf16_bits(x), device), to_dev(O.f32_to_bf16_bits(w), device), (N + 7) // 8 * 8, MI)
+    torch.cuda.synchronize()
+    assert np.array_equal(bits(y[:, 2 * MI:].contiguous()), gu[:, 2 * MI:])
+    # silu runs on hardware exp2 and reciprocal: one bf16 step where a value lies at a rounding boundary
+    ref, got = O.bf16_bits_to_f32(O.swiglu_bf16(gu, MI)), O.bf16_bits_to_f32(bits(act))
+    assert np.all(np.abs(got - ref) <= np.maximum(np.abs(ref) * 2.0 ** -6, 1e-30))
+    assert np.mean(got != ref) < 0.01
