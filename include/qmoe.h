@@ -99,6 +99,11 @@ size_t qmoe_route_group_workspace(int R, int E);
 int qmoe_route_group(const void* ids, int R, int E, void* counts, void* ends, void* order, void* inverse,
                      int BM, void* tile_expert, void* tile_row0, void* tile_rows, void* tile_count,
                      void* workspace, size_t workspace_bytes, void* stream);
+/* qmoe_router_topk followed by qmoe_route_group of its ids (one launch for a
+ * few tokens); arguments as theirs, workspace qmoe_route_group_workspace(T k, E). */
+int qmoe_route_tokens(const void* logits, int T, int E, int k, void* idx_out, void* w_out, void* counts, void* ends,
+                      void* order, void* inverse, int BM, void* tile_expert, void* tile_row0, void* tile_rows,
+                      void* tile_count, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- Fused decode expert block for B = 1..4 tokens (FnLayer._moe b == 1
  *      branch, fnx/engine.py:1859-1891, r152 flags): router, gate_up of the

@@ -12,6 +12,7 @@
 //                then one workgroup scans the totals into counts/ends (int64,
 //                inclusive cumsum = group_list) and emits the grouped GEMM's
 //                row-tile table (expert, first row, rows).
+//   (up to 8192 ids over 1024 experts: all of it in one workgroup instead)
 //   3. scatter : one wave per chunk (run bases = expert start + chunk offset)
 //                walks its ids in flat order; an id's rank
 //                among equal ids before it in the same wave step comes from
@@ -339,6 +340,115 @@ __global__ __launch_bounds__(64) void route_scatter_kernel(const int64_t* __rest
   }
 }
 
+// Small batches: the whole grouping in one workgroup, and for a few tokens
+// (KPL > 0) the router as well, wave w routing tokens w, w + 16, ... A launch
+// costs more here than its work: the four grouping launches and the router's
+// take 25 us at 23 tokens, this one 9.
+// Wave w owns a contiguous run of flat ids and ranks them in flat order (ballots
+// within a step of 64, an LDS count per expert between steps); the per-wave
+// counts then become each wave's offset within the expert's run, so the order
+// is the stable one of the separate launches.
+constexpr int kSmallSteps = 8;       // steps of 64 ids per wave, at most
+constexpr int kSmallIds = 64 * 16 * kSmallSteps;
+constexpr int kSmallExperts = 1024;  // one thread per expert
+constexpr int kSmallTokens = 32;     // tokens routed here: two per wave
+
+template <int KPL>
+__global__ __launch_bounds__(1024) void route_small_kernel(const uint16_t* __restrict__ logits,
+                                                           const int64_t* __restrict__ ids, int T, int k, int R, int E,
+                                                           int64_t* __restrict__ idx_out, uint16_t* __restrict__ w_out,
+                                                           int64_t* __restrict__ counts, int64_t* __restrict__ ends,
+                                                           int64_t* __restrict__ order, int64_t* __restrict__ inverse,
+                                                           int BM, int max_tiles, int* __restrict__ tile_expert,
+                                                           int* __restrict__ tile_row0, int* __restrict__ tile_rows,
+                                                           int* __restrict__ tile_count) {
+  __shared__ uint16_t s_run[kScanWaves][kSmallExperts];  // ids per wave and expert, then the wave's offset
+  __shared__ int s_tot[kSmallExperts];
+  __shared__ int s_start[kSmallExperts];
+  __shared__ TileScratch ts;
+  __shared__ int s_ids[KPL > 0 ? kSmallTokens * QMOE_KMAX : 1];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int e = lane; e < E; e += 64) s_run[wave][e] = 0;  // this wave's row
+  const int chunk = (R + 64 * kScanWaves - 1) / (64 * kScanWaves);  // steps of 64 ids per wave
+  int ev[kSmallSteps], rank[kSmallSteps];
+  if constexpr (KPL > 0) {
+    __shared__ int s_idx[kScanWaves][QMOE_KMAX];
+    __shared__ float s_w[kScanWaves][QMOE_KMAX];
+    for (int t = wave; t < T; t += kScanWaves) {
+      wave_topk_softmax<KPL>(logits + (size_t)t * E, E, k, s_idx[wave], s_w[wave]);
+      if (lane < k) {
+        const int e = s_idx[wave][lane];
+        s_ids[t * k + lane] = e;
+        idx_out[(size_t)t * k + lane] = e;
+        w_out[(size_t)t * k + lane] = (uint16_t)f32_to_bf16(s_w[wave][lane]);
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int q = 0; q < kSmallSteps; ++q) {
+    const int f = (wave * chunk + q) * 64 + lane;
+    ev[q] = -1;
+    if (q < chunk && f < R) {
+      if constexpr (KPL > 0) {
+        ev[q] = s_ids[f];
+      } else {
+        const int64_t v = ids[f];
+        ev[q] = (v >= 0 && v < E) ? (int)v : -1;
+      }
+    }
+  }
+  const int nbits = 32 - __builtin_clz((unsigned)max(E - 1, 1));
+#pragma unroll
+  for (int q = 0; q < kSmallSteps; ++q) {
+    if (q >= chunk) break;
+    const int key = (ev[q] >= 0) ? ev[q] : (1 << nbits);
+    uint64_t same = ~0ull;
+    for (int b = 0; b <= nbits; ++b) {
+      const bool bit = (key >> b) & 1;
+      const uint64_t bal = __ballot(bit);
+      same &= bit ? bal : ~bal;
+    }
+    rank[q] = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+    const bool last = (lane == 63) || ((same >> (lane + 1)) == 0ull);
+    // every lane of the wave reads the count before the last of each expert advances it
+    if (ev[q] >= 0) rank[q] += s_run[wave][ev[q]];
+    __builtin_amdgcn_wave_barrier();
+    if (ev[q] >= 0 && last) s_run[wave][ev[q]] = (uint16_t)(rank[q] + 1);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  int tot = 0;
+  if (tid < E) {
+#pragma unroll
+    for (int q = 0; q < kScanWaves; ++q) {
+      const int c = s_run[q][tid];
+      s_run[q][tid] = (uint16_t)tot;
+      tot += c;
+    }
+  }
+  int all = 0;
+  const int start = block_excl_scan(tot, ts.w, &all);
+  if (tid < E) {
+    s_tot[tid] = tot;
+    s_start[tid] = start;
+    counts[tid] = tot;
+    ends[tid] = start + tot;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kSmallSteps; ++q) {
+    const int f = (wave * chunk + q) * 64 + lane;
+    if (q < chunk && f < R) {
+      const int pos = ev[q] >= 0 ? s_start[ev[q]] + s_run[wave][ev[q]] + rank[q] : -1;
+      inverse[f] = pos;
+      if (pos >= 0) order[pos] = f;
+    }
+  }
+  if (tile_expert != nullptr)
+    write_row_tiles(s_tot, s_start, E, BM, max_tiles, tile_expert, tile_row0, tile_rows, tile_count, ts);
+}
+
 // Row-tile table of the grouped GEMM from an inclusive cumulative group list
 // (the grouped_matmul entry point, where rows are already expert-sorted).
 __global__ __launch_bounds__(1024) void tiles_from_ends_kernel(const int64_t* __restrict__ ends, int E, int BM,
@@ -409,6 +519,13 @@ int qmoe_route_group(const void* ids, int R, int E, void* counts, void* ends, vo
   if (workspace_bytes < qmoe_route_group_workspace(R, E)) return QMOE_EWORKSPACE;
   const int nchunks = host_ceil_div(R, kChunk);
   hipStream_t st = (hipStream_t)stream;
+  if (R <= kSmallIds && E <= kSmallExperts) {
+    hipLaunchKernelGGL(route_small_kernel<0>, dim3(1), dim3(1024), 0, st, (const uint16_t*)nullptr, (const int64_t*)ids,
+                       0, 0, R, E, (int64_t*)nullptr, (uint16_t*)nullptr, (int64_t*)counts, (int64_t*)ends,
+                       (int64_t*)order, (int64_t*)inverse, BM, qmoe_max_row_tiles(R, E, BM < 1 ? 1 : BM),
+                       (int*)tile_expert, (int*)tile_row0, (int*)tile_rows, (int*)tile_count);
+    return (int)hipGetLastError();
+  }
   int* hist = (int*)workspace;
   const size_t lds = (size_t)E * sizeof(int);
   hipLaunchKernelGGL(route_count_kernel, dim3(nchunks), dim3(64), lds, st, (const int64_t*)ids, R, E, hist);
@@ -420,6 +537,30 @@ int qmoe_route_group(const void* ids, int R, int E, void* counts, void* ends, vo
                      (const int*)hist, (const int64_t*)counts, (const int64_t*)ends, (int64_t*)order,
                      (int64_t*)inverse);
   return (int)hipGetLastError();
+}
+
+int qmoe_route_tokens(const void* logits, int T, int E, int k, void* idx_out, void* w_out, void* counts, void* ends,
+                      void* order, void* inverse, int BM, void* tile_expert, void* tile_row0, void* tile_rows,
+                      void* tile_count, void* workspace, size_t workspace_bytes, void* stream) {
+  if (T < 1 || E < 1 || E > 1024 || k < 1 || k > QMOE_KMAX || k > E || (tile_expert != nullptr && BM < 1))
+    return QMOE_EINVAL;
+  if ((long)T * k > 0x7fffffffL) return QMOE_EINVAL;
+  if (workspace_bytes < qmoe_route_group_workspace(T * k, E)) return QMOE_EWORKSPACE;
+  if (T <= kSmallTokens) {
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, (hipStream_t)stream, (const uint16_t*)logits,
+                         (const int64_t*)nullptr, T, k, T * k, E, (int64_t*)idx_out, (uint16_t*)w_out,
+                         (int64_t*)counts, (int64_t*)ends, (int64_t*)order, (int64_t*)inverse, BM,
+                         qmoe_max_row_tiles(T * k, E, BM < 1 ? 1 : BM), (int*)tile_expert, (int*)tile_row0,
+                         (int*)tile_rows, (int*)tile_count);
+      return (int)hipGetLastError();
+    };
+    return E <= 512 ? go(route_small_kernel<8>) : go(route_small_kernel<16>);
+  }
+  const int rc = qmoe_router_topk(logits, idx_out, w_out, T, E, k, stream);
+  if (rc) return rc;
+  return qmoe_route_group(idx_out, T * k, E, counts, ends, order, inverse, BM, tile_expert, tile_row0, tile_rows,
+                          tile_count, workspace, workspace_bytes, stream);
 }
 
 int qmoe_tiles_from_ids(const void* ids, int k, int E, void* tile_expert, void* tile_row0, void* tile_rows,

@@ -51,6 +51,7 @@ SIGNATURES = {
     "qmoe_route_group_workspace": (Z, [I, I]),
     "qmoe_max_row_tiles": (I, [I, I, I]),
     "qmoe_route_group": (I, [P, I, I, P, P, P, P, I, P, P, P, P, P, Z, P]),
+    "qmoe_route_tokens": (I, [P, I, I, I, P, P, P, P, P, P, I, P, P, P, P, P, Z, P]),
     "qmoe_tiles_from_ends": (I, [P, I, I, I, P, P, P, P, P]),
     "qmoe_tiles_from_ids": (I, [P, I, I, P, P, P, P, P]),
     "qmoe_gemm_tile_rows": (I, []),

@@ -24,7 +24,7 @@ import os
 import torch
 
 from . import _lib
-from .ops import grouped_matmul, route_group, router_topk, weight_quant_batchmatmul
+from .ops import grouped_matmul, route_tokens, weight_quant_batchmatmul
 
 BF16 = torch.bfloat16
 DECODE_MAX_TOKENS = 4
@@ -407,10 +407,9 @@ def moe_prefill(x, logits, exp_gu, exp_dn, topk, shared=None, return_routing=Fal
     dev = x.device
     MI = exp_dn.K
     E = exp_gu.E
-    idx, w = router_topk(logits, topk)
     L = _lib.lib()
     bm = L.qmoe_moe_tile_rows(T * topk, E, H, MI, exp_gu.gs, exp_dn.gs)
-    counts, ends, order, inverse, tiles, mt = route_group(idx, E, with_tiles=True, tile_rows=bm)
+    idx, w, counts, ends, order, inverse, tiles, mt = route_tokens(logits, topk, bm)
     out = torch.empty((T, H), dtype=BF16, device=dev)
     ws = _lib.workspace(dev, L.qmoe_moe_prefill_workspace(T, topk, H, MI))
     sh = shared.contiguous() if shared is not None else None

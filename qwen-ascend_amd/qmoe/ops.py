@@ -6,8 +6,9 @@
   ``split_item=3, group_type=0`` (``fnx/engine.py:712-716, 744-753``).
 * :func:`swiglu` — ``npu_swiglu(gu.float(), dim=-1).to(torch.bfloat16)``
   (``fnx/engine.py:1827, 1866``).
-* :func:`router_topk`, :func:`route_group` — the router and grouping glue of
-  ``FnLayer._moe`` (``fnx/engine.py:1810-1823, 1832-1843``) on the GPU.
+* :func:`router_topk`, :func:`route_group`, :func:`route_tokens` (both) — the
+  router and grouping glue of ``FnLayer._moe`` (``fnx/engine.py:1810-1823,
+  1832-1843``) on the GPU.
 
 All launch HIP kernels from libqmoe.so on the current stream, allocate only
 through torch, and never synchronise, so they can be captured in a graph.
@@ -239,3 +240,27 @@ def route_group(idx, E, with_tiles=False, tile_rows=None):
     if with_tiles:
         return counts, ends, order, inverse, tiles, mt
     return counts, ends, order, inverse
+
+
+def route_tokens(logits, k, tile_rows):
+    """:func:`router_topk` and :func:`route_group` of its ids with the row-tile
+    table: (idx, w, counts, ends, order, inverse, tiles, max tiles)."""
+    if logits.dim() != 2 or logits.dtype != BF16:
+        raise RuntimeError("logits must be bf16 [T, E]")
+    _cuda(logits)
+    logits = logits.contiguous()
+    T, E = logits.shape
+    R, dev = T * k, logits.device
+    w = torch.empty((T, k), dtype=BF16, device=dev)
+    ints = torch.empty((2 * E + 3 * R,), dtype=torch.int64, device=dev)
+    counts, ends, idx, order, inverse = ints.split((E, E, R, R, R))
+    idx = idx.view(T, k)
+    L = _lib.lib()
+    bm, mt, tiles = _tile_table(R, E, dev, tile_rows)
+    ws = _lib.workspace(dev, L.qmoe_route_group_workspace(R, E))
+    t0 = tiles.data_ptr()
+    _lib.check(L.qmoe_route_tokens(logits.data_ptr(), T, E, k, idx.data_ptr(), w.data_ptr(), counts.data_ptr(),
+                                   ends.data_ptr(), order.data_ptr(), inverse.data_ptr(), bm, t0, t0 + 4 * mt,
+                                   t0 + 8 * mt, t0 + 12 * mt, ws.data_ptr(), ws.numel(), _lib.stream_of(logits)),
+               "route_tokens")
+    return idx, w, counts, ends, order, inverse, tiles, mt

@@ -75,3 +75,48 @@ def test_route_group_ignores_invalid_ids(device):
     inv = inverse.cpu().numpy()
     assert inv[2] == -1 and inv[4] == -1
     assert order.cpu().numpy()[:4].tolist() == [5, 0, 3, 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,k,bm", [(1, 512, 10, 12), (17, 40, 8, 12), (32, 1000, 16, 128), (33, 512, 10, 12),
+                                      (819, 64, 10, 12), (820, 64, 10, 128)])
+def test_route_tokens(device, T, E, k, bm):
+    """Router and grouping in one call, at the edges of the one-workgroup forms
+    (32 tokens, 8192 ids): ids, stable order and the row-tile table."""
+    from qmoe.ops import route_tokens
+    log(f"route_tokens T={T} E={E} k={k} bm={bm}")
+    lg = bf16_normal((T, E), T + E)
+    lg[:, 0] = 0x4200                           # one expert every token picks
+    lg[0, 3] = lg[0, E - 1] = 0x4200            # ties: lower id first
+    idx, w, counts, ends, order, inverse, tiles, mt = route_tokens(to_dev(lg, device), k, bm)
+    torch.cuda.synchronize()
+    ridx, _ = O.router(lg, k)
+    rc, re, ro, ri = O.group_routing(ridx, E)
+    for got, ref in ((idx, ridx), (counts, rc), (ends, re), (order, ro), (inverse, ri)):
+        assert np.array_equal(got.cpu().numpy(), ref)
+    from parity import assert_rounds_exactly
+    assert_rounds_exactly(w, O.router_weights_exact(lg, ridx), None, f"router weights T={T}")
+    t = tiles.cpu().numpy()
+    n = int(t[3 * mt])
+    assert n == int(np.sum((rc + bm - 1) // bm))
+    covered = np.zeros(T * k, dtype=np.int64)
+    for e_, a, c in zip(t[:n], t[mt:mt + n], t[2 * mt:2 * mt + n]):
+        assert 0 < c <= bm and re[e_] - rc[e_] <= a and a + c <= re[e_]
+        covered[a:a + c] += 1
+    assert np.all(covered == 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("R,E", [(1, 1), (100, 7), (8192, 1024), (8193, 1024)])
+def test_route_group_ids_outside(device, R, E):
+    """Ids outside [0, E) are neither counted nor placed, on both forms."""
+    from qmoe import route_group
+    ids = np.random.default_rng(R).integers(-2, E + 2, size=(R,)).astype(np.int64)
+    counts, ends, order, inverse = (t.cpu().numpy() for t in route_group(to_dev(ids, device), E))
+    ok = (ids >= 0) & (ids < E)
+    rc = np.bincount(ids[ok], minlength=E)
+    ro = np.flatnonzero(ok)[np.argsort(ids[ok], kind="stable")]
+    ri = np.full(R, -1)
+    ri[ro] = np.arange(ro.size)
+    assert np.array_equal(counts, rc) and np.array_equal(ends, np.cumsum(rc))
+    assert np.array_equal(order[:ro.size], ro) and np.array_equal(inverse, ri)
