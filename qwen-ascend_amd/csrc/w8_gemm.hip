@@ -18,8 +18,8 @@
 //
 // Few rows or few tiles: bf16 MFMA (16x16x32), K split over a workgroup's
 // waves, weights streamed into registers.
-// Else: the same MFMA on 128 x 64 output tiles, the operands streaming
-// through an LDS ring of chunks. int8 values are exact in bf16, so the MFMA sums
+// Else: the same MFMA on 128 x 128 output tiles (128 x 64 for groups that are
+// not whole 64-k chunks), the operands streaming through an LDS ring of chunks. int8 values are exact in bf16, so the MFMA sums
 // x * q exactly per product with fp32 accumulation; after each scale group
 // the group's partial sums are scaled by S[g, n] and added to the output
 // accumulators.
@@ -152,6 +152,10 @@ typedef float f32x4_v __attribute__((ext_vector_type(4)));
 
 constexpr int kBK = 32;                     // k per MFMA step
 
+// four bf16 results as one 8-byte store (y rows may start at any element)
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+QMOE_DEV void store_bf16x4(uint16_t* p, uint32_t lo, uint32_t hi) { *reinterpret_cast<u32x2_a2*>(p) = u32x2_a2{lo, hi}; }
+
 QMOE_DEV uint32_t i8_to_bf16_bits(uint32_t word, int byte) {
   return __float_as_uint((float)(int)(int8_t)(word >> (8 * byte))) >> 16;
 }
@@ -163,6 +167,15 @@ QMOE_DEV uint32_t i8_to_bf16_bits(uint32_t word, int byte) {
 QMOE_DEV void lds_write8_untracked(void* p, uint32_t lo, uint32_t hi) {
   const unsigned a = (unsigned)(size_t)(__attribute__((address_space(3))) char*)p;
   asm volatile("ds_write_b64 %0, %1" ::"v"(a), "v"(make_uint2(lo, hi)) : "memory");
+}
+
+// An 8-byte LDS read the compiler does not track (an ordinary one would wait for
+// the DMAs in flight); waits for its own result.
+QMOE_DEV uint2 lds_read8_untracked(const void* p) {
+  const unsigned a = (unsigned)(size_t)(__attribute__((address_space(3))) const char*)p;
+  uint2 v;
+  asm volatile("ds_read_b64 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(a) : "memory");
+  return v;
 }
 
 // The weight fragments of a chunk's two MFMA steps (two per step, 16 columns
@@ -620,8 +633,8 @@ __global__ __launch_bounds__(64 * NW) void w8a16_skinny_kernel(const uint16_t* _
       a.w += b.w;
     }
     if (n0 + c < N)
-      *reinterpret_cast<uint2*>(y + (size_t)(m0 + row) * N + n0 + c) =
-          make_uint2(f32_to_bf16(a.x) | (f32_to_bf16(a.y) << 16), f32_to_bf16(a.z) | (f32_to_bf16(a.w) << 16));
+      store_bf16x4(y + (size_t)(m0 + row) * N + n0 + c, f32_to_bf16(a.x) | (f32_to_bf16(a.y) << 16),
+                   f32_to_bf16(a.z) | (f32_to_bf16(a.w) << 16));
   }
 }
 
@@ -677,6 +690,279 @@ int launch_w8_few_tiles(const void* x, const void* w, const void* scale, void* y
   if (live == 2) return launch_w8_skinny<2, 16, 1, 4>(x, w, scale, y, M, K, N, gs, st);
   if (live == 3) return launch_w8_skinny<3, 8, 1, 4>(x, w, scale, y, M, K, N, gs, st);
   return launch_w8_skinny<4, 8, 1, 4>(x, w, scale, y, M, K, N, gs, st);
+}
+
+// ---------------------------------------------------------------- many tiles, 64-k groups: conversion in registers
+//
+// 128 x 128 output tiles, 4 waves (2 x 2) of 64 x 64: 4 x 4 MFMA tiles each. K
+// runs in 64-k chunks (x rows and raw int8 weight rows, with the bf16 scale row
+// of the chunk's group) through a ring of three LDS slots by buffer-resource
+// global->LDS DMA, two chunks ahead; one barrier per chunk. A lane reads, for
+// each of its 8 k rows of a step, the 4 bytes of its columns 4 i16 .. 4 i16 + 3,
+// and makes the four B fragments of the step itself: one conversion per value
+// and one v_perm per pair (int8 is exact in bf16), between the MFMAs of the
+// fragment before. So the weights are neither written back to LDS nor read a
+// second time, and no conversion stands in the chunk's chain.
+// LDS: x row r holds k-piece p at p ^ (r & 7); weight row r sits at r ^ 1 for
+// odd r / 8 and its words at w ^ 16 for odd r / 16, so the four 16-word pieces a
+// wave reads at once lie in different banks.
+//
+// What bounds it: VALU and MFMA issue. With one wave per SIMD a chunk costs the
+// wave about 100 conversion and 32 scaling operations at 5 cycles each beside 512
+// cycles of MFMA; issued in blocks rather than behind the MFMAs, with the seven
+// DMA instructions together (350 cycles) and the chunk's LDS reads ahead of it
+// (415), it took 2130. 2048 x 8192 at 512 rows 39.1 -> 24.5 us (700 TFLOP/s), at
+// 1024 73.0 -> 40.6 (847), 4096 x 4096 at 4096 rows 273 -> 176 (781), against 128
+// x 64 tiles that converted through LDS. A deeper ring changes nothing (4 and 6
+// slots: 31.2 and 31.9 us where 3 took 30.6).
+struct W8Reg {
+  static constexpr int BM = 128, BN = 128, KC = 64, RING = 3;
+  static constexpr int A_BYTES = BM * KC * 2, B_BYTES = KC * BN, S_BYTES = 1024;  // scales: one DMA instruction, 256 bytes used
+  static constexpr int SLOT = A_BYTES + B_BYTES + S_BYTES;
+  static constexpr int IPC = 4 + 2 + 1;  // DMA instructions per wave and chunk: x, weights, scales
+  static constexpr int LDS = RING * SLOT;
+};
+
+template <int KS, int CPG>
+__global__ __launch_bounds__(kThreads * KS, 2) void w8a16_reg_kernel(const uint16_t* __restrict__ x,
+                                                                const int8_t* __restrict__ w,
+                                                                const uint16_t* __restrict__ s,
+                                                                uint16_t* __restrict__ y, int M, int K, int N, int gs) {
+  using T = W8Reg;
+  constexpr int RING = T::RING;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  const int ntn = (N + T::BN - 1) / T::BN;
+  const int ntiles = ((M + T::BM - 1) / T::BM) * ntn;
+  const int tile = xcd_remap(blockIdx.x, gridDim.x);
+  if (tile >= ntiles) return;
+  const int nrt = ntiles / ntn;  // row tiles of a column tile side by side on one XCD: its weights come through one L2
+  const int m0 = (tile % nrt) * T::BM, n0 = (tile / nrt) * T::BN;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) & 3);
+  const int ks = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads);
+  unsigned char* ring = lds + ks * T::LDS;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int i16 = lane & 15, kb = lane >> 4;
+
+  constexpr int kRsrcWord3 = 0x00020000;
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void*)x, (short)0, M * K * 2, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, K * N, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rsrc_s =
+      __builtin_amdgcn_make_buffer_rsrc((void*)s, (short)0, (K / gs) * N * 2, kRsrcWord3);
+  // this wave group's run of chunks: whole scale groups of cpg chunks, the same number for each
+  const int cpg = CPG != 0 ? CPG : gs / T::KC;
+  const int nch = K / T::KC / KS, c0 = ks * nch;
+  uint32_t aoff[4], boff[2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = 8 * (4 * q + wave) + (lane >> 3);
+    aoff[q] = 2u * ((uint32_t)min(m0 + r, M - 1) * (uint32_t)K + 8u * (uint32_t)((lane & 7) ^ (r & 7)));
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int b = 4 * q + wave;  // 8 weight rows
+    boff[q] = (uint32_t)(8 * b + ((lane >> 3) ^ (b & 1))) * (uint32_t)N +
+              (uint32_t)(n0 + 16 * ((lane & 7) ^ (4 * ((b >> 1) & 1))));
+  }
+  // scales: every wave writes the same row; lanes past it read beyond the
+  // resource's extent, which gives zeros and no traffic
+  const uint32_t soff = lane < 16 ? 2u * (uint32_t)(n0 + 8 * lane) : 0x80000000u;
+  // DMA instruction j of a chunk: 0, 1 weights, 2 .. 5 x, 6 scales
+  // (srow: byte offset of the scale row of the chunk's group)
+  auto issue_one = [&](int j, int c, int slot, int srow) {
+    unsigned char* base = ring + slot * T::SLOT;
+    const int k0 = (c0 + c) * T::KC;
+    if (j < 2) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc_b, (__attribute__((address_space(3))) void*)(base + T::A_BYTES + (4 * j + wave) * 1024), 16, (int)boff[j],
+          k0 * N, 0, 0);
+    } else if (j < 6) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rsrc_a, (__attribute__((address_space(3))) void*)(base + (4 * (j - 2) + wave) * 1024), 16, (int)aoff[j - 2],
+          k0 * 2, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_s, (__attribute__((address_space(3))) void*)(base + T::A_BYTES + T::B_BYTES),
+                                               16, (int)soff, srow, 0, 0);
+    }
+  };
+
+  f32x4_v acc[4][4], accg[4][4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int f = 0; f < 4; ++f) acc[t][f] = f32x4_v{0.f, 0.f, 0.f, 0.f};
+  // this lane's LDS offsets: x row i16 of row tile 0 (its pieces by step), its
+  // word of even and odd weight rows
+  const int arow = (wm * 64 + i16) * 128;
+  const int bword = 4 * ((16 * wn + i16) ^ (16 * (kb >> 1))) + 8 * kb * 128;
+  const int beven = T::A_BYTES + bword + (kb & 1) * 128, bodd = T::A_BYTES + bword - (kb & 1) * 128;
+
+#pragma unroll
+  for (int c = 0; c < RING - 1; ++c)
+    {
+      const int cc = min(c, nch - 1);
+#pragma unroll
+      for (int j = 0; j < T::IPC; ++j) issue_one(j, cc, c, (c0 + cc) * T::KC / gs * N * 2);
+    }
+  // the current ring slot; the chunk DMA'd next (the run's last one again past
+  // its end, into a slot that is not read any more), its scale row and its
+  // group's chunks left, counted
+  int slot = 0, inext = min(RING - 1, nch - 1);
+  int irow = (c0 + inext) * T::KC / gs * N * 2, ileft = cpg - (c0 + inext) % cpg;
+  // one chunk; FIRST / LAST: it starts / ends a run of group sums
+  auto chunk = [&](auto first_c, auto last_c) {
+    constexpr bool FIRST = decltype(first_c)::value != 0, LAST = decltype(last_c)::value != 0;
+    wait_vm_lgkm0<(RING - 2) * T::IPC>();
+    // every wave is past the chunk before: its slot takes the chunk RING - 1 ahead
+    barrier_no_fence();
+    const unsigned char* base = ring + slot * T::SLOT;
+    uint32_t bw[2][8];
+    bf16x8_v af[2][4];
+    auto read_words = [&](int st) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        bw[st][i] = *reinterpret_cast<const uint32_t*>(base + ((i & 1) ? bodd : beven) + (32 * st + i) * 128);
+    };
+    auto read_x = [&](int st, int t) {
+      af[st][t] = *reinterpret_cast<const bf16x8_v*>(base + arow + t * 16 * 128 + (((4 * st + kb) ^ (i16 & 7)) << 4));
+    };
+    // pair i of fragment n (step n / 4, column n % 4)
+    auto pair = [&](int n, int i) -> uint32_t {
+      const float lo = (float)(int)(int8_t)(bw[n >> 2][2 * i] >> (8 * (n & 3)));
+      const float hi = (float)(int)(int8_t)(bw[n >> 2][2 * i + 1] >> (8 * (n & 3)));
+      return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+    };
+    read_words(0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) read_x(0, t);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t cur[4], nxt[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cur[i] = pair(0, i);
+    __builtin_amdgcn_sched_barrier(0);
+    // Behind each MFMA, in its shadow: a pair of the next fragment (three VALU
+    // operations), step 1's reads behind step 0's first fragment, one DMA
+    // instruction of the chunk to come per fragment (issued together they held
+    // the wave for 350 cycles) and, in a group's last chunk, the scaled sums of
+    // the columns that are complete. sched_barrier keeps this order.
+    uint2 sv{};
+    float sc = 0.f;
+    auto scaled = [&](int f, int t) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[t][f][r] = __builtin_fmaf(accg[t][f][r], sc, acc[t][f][r]);
+    };
+    auto scale_of = [&](int f) {
+      const uint32_t v = f < 2 ? sv.x : sv.y;
+      return __uint_as_float((f & 1) ? (v & 0xffff0000u) : (v << 16));
+    };
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      const bf16x8_v b = __builtin_bit_cast(bf16x8_v, make_uint4(cur[0], cur[1], cur[2], cur[3]));
+      if (LAST && n >= 5) sc = scale_of(n - 5);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        accg[t][n & 3] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            af[n >> 2][t], b, (FIRST && n < 4) ? f32x4_v{0.f, 0.f, 0.f, 0.f} : accg[t][n & 3], 0, 0, 0);
+        if (n < 7) nxt[t] = pair(n + 1, t);
+        if (n == 0 && t == 0) read_words(1);
+        if (n == 0 && t > 1) {
+          read_x(1, 2 * t - 4);
+          read_x(1, 2 * t - 3);
+        }
+        if (n < 7 && t == 3) issue_one(n, inext, slot == 0 ? RING - 1 : slot - 1, irow);
+        if (LAST && n >= 5) scaled(n - 5, t);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (LAST && n == 3) sv = lds_read8_untracked(base + T::A_BYTES + T::B_BYTES + 2 * (64 * wn + 4 * i16));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cur[i] = nxt[i];
+    }
+    if (LAST) {
+      sc = scale_of(3);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) scaled(3, t);
+    }
+  };
+  auto next_chunk = [&]() {
+    slot = slot + 1 == RING ? 0 : slot + 1;
+    if (inext + 1 < nch) {
+      ++inext;
+      if (--ileft == 0) {
+        ileft = cpg;
+        irow += 2 * N;
+      }
+    }
+  };
+  for (int c = 0; c < nch; c += cpg) {
+    if constexpr (CPG == 1) {
+      chunk(W8C<1>{}, W8C<1>{});
+      next_chunk();
+    } else {
+      chunk(W8C<1>{}, W8C<0>{});
+      next_chunk();
+      if constexpr (CPG == 0) {
+        for (int i = 2; i < cpg; ++i) {
+          chunk(W8C<0>{}, W8C<0>{});
+          next_chunk();
+        }
+      }
+      chunk(W8C<0>{}, W8C<1>{});
+      next_chunk();
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the DMA past the end
+  if constexpr (KS > 1) {
+    // the second group's tile through LDS
+    float4* part = reinterpret_cast<float4*>(lds);  // [4][4][256 threads]
+    const int gt = threadIdx.x % kThreads;
+    __syncthreads();
+    if (ks > 0) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+          part[(4 * t + f) * kThreads + gt] = make_float4(acc[t][f][0], acc[t][f][1], acc[t][f][2], acc[t][f][3]);
+    }
+    __syncthreads();
+    if (ks > 0) return;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const float4 v = part[(4 * t + f) * kThreads + gt];
+        acc[t][f] += f32x4_v{v.x, v.y, v.z, v.w};
+      }
+  }
+  // lane holds columns 4 i16 .. + 3 for rows 4 kb .. + 3 of each row tile
+  const int col = n0 + 64 * wn + 4 * i16;
+  if (col >= N) return;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = m0 + 64 * wm + 16 * t + 4 * kb + r;
+      if (row < M)
+        store_bf16x4(y + (size_t)row * N + col, pk_bf16(acc[t][0][r], acc[t][1][r]), pk_bf16(acc[t][2][r], acc[t][3][r]));
+    }
+}
+
+template <int KS, int CPG>
+int launch_w8_reg(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs, hipStream_t st) {
+  int dev = 0;
+  hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return (int)err;
+  if (dev < 0 || dev >= 64) return QMOE_EINVAL;
+  static bool attr_set[64] = {};
+  if (!attr_set[dev]) {
+    err = hipFuncSetAttribute((const void*)w8a16_reg_kernel<KS, CPG>, hipFuncAttributeMaxDynamicSharedMemorySize, KS * W8Reg::LDS);
+    if (err != hipSuccess) return (int)err;
+    attr_set[dev] = true;
+  }
+  const long blocks = ((long)host_ceil_div(M, W8Reg::BM) * host_ceil_div(N, W8Reg::BN) + 7) / 8 * 8;
+  if (blocks > 0x7fffffffL) return QMOE_EINVAL;
+  hipLaunchKernelGGL((w8a16_reg_kernel<KS, CPG>), dim3((unsigned)blocks), dim3(kThreads * KS), KS * W8Reg::LDS, st, (const uint16_t*)x,
+                     (const int8_t*)w, (const uint16_t*)scale, (uint16_t*)y, M, K, N, gs);
+  return (int)hipGetLastError();
 }
 
 template <class T>
@@ -757,14 +1043,27 @@ int qmoe_w8a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
                          int group_size, void* stream) {
   if (!w8_mfma_ok(x, w, M, K, N, group_size)) return QMOE_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  // 128 x 64 tiles (64-k chunks when the group size allows: twice the MFMA work
-  // per barrier) above 256 rows where they still give every CU a workgroup,
-  // else the skinny kernel. At 2048 x 8192 the tiles take 28.5 us for 129 to
-  // 256 rows, the skinny kernel 20.1 to 24.9; at 512 rows 39.1 against 46.5.
-  const long tiles128 = (long)((M + 127) / 128) * ((N + 63) / 64);
-  if (M <= 256 || tiles128 < 256) return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, st);
-  if (group_size % 64 == 0 && K % 64 == 0)
-    return launch_w8_mfma<W8Tile<128, 64, 64, 3>>(x, w, scale, y, M, K, N, group_size, st);
+  // Groups of whole 64-k chunks: 128 x 128 tiles from 128 of them on. At 2048 x
+  // 8192 they take 23.1 us for 256 rows and the skinny kernel 29.4 from cold
+  // weights; with 64 tiles 22.4 against 15.2 (512 rows, 2048 x 2048). Up to one
+  // tile per CU K is split over two groups of waves where both get whole scale
+  // groups (4096 x 4096 at 512 rows 42.5 against 53.4 us); beyond, two workgroups
+  // share a CU instead (2048 x 8192 at 1024 rows 40.6 against 45.8).
+  const long tiles = (long)host_ceil_div(M, 128) * host_ceil_div(N, 128);
+  if (group_size % 64 == 0) {
+    if (tiles < 128) return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, st);
+    auto go = [&](auto ks) {
+      constexpr int KS = decltype(ks)::value;
+      if (group_size == 64) return launch_w8_reg<KS, 1>(x, w, scale, y, M, K, N, group_size, st);
+      if (group_size == 128) return launch_w8_reg<KS, 2>(x, w, scale, y, M, K, N, group_size, st);
+      return launch_w8_reg<KS, 0>(x, w, scale, y, M, K, N, group_size, st);
+    };
+    return tiles <= 256 && K / group_size % 2 == 0 ? go(W8C<2>{}) : go(W8C<1>{});
+  }
+  // other groups: 128 x 64 tiles of 32-k chunks above 256 rows where they give
+  // every CU a workgroup
+  if (M <= 256 || (long)host_ceil_div(M, 128) * host_ceil_div(N, 64) < 256)
+    return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, st);
   return launch_w8_mfma<W8Tile<128, 64, 32, 4>>(x, w, scale, y, M, K, N, group_size, st);
 }
 

@@ -72,6 +72,25 @@ def test_w8a16_few_tiles(device, M, K, N, gs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,gs", [
+    (200, 128, 8208, 64), (257, 64, 8080, 64),      # K split in two; one chunk, ragged rows and columns
+    (130, 512, 8192, 128), (640, 384, 8192, 128),   # 2-chunk groups: split and not
+    (1000, 768, 2064, 256), (300, 192, 6544, 192),  # longer groups
+])
+def test_w8a16_register_tiles(device, M, K, N, gs):
+    """128 x 128 tiles with the conversion in registers: each group length, K
+    whole and split, partial tiles, scales off a 16-byte boundary."""
+    from qmoe import weight_quant_batchmatmul
+    log(f"w8a16 register tiles M={M} K={K} N={N} gs={gs}")
+    x, q, S = w8_case(M, K, N, gs, M + K)
+    sd = torch.empty(K // gs * N + 1, dtype=torch.bfloat16, device=device)[1:].view(K // gs, N)
+    sd.copy_(to_dev(S, device))
+    y = weight_quant_batchmatmul(to_dev(x, device), to_dev(q, device), sd, antiquant_group_size=gs)
+    torch.cuda.synchronize()
+    check(bits(y), x, q, S, gs, f"w8a16 register tiles M={M}")
+
+
+@pytest.mark.gpu
 def test_w8a16_small_group_gemv(device):
     """gs = 8 (a 4-row run per thread stays in one group) on the GEMV path."""
     from qmoe import weight_quant_batchmatmul
