@@ -56,7 +56,7 @@ int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
  *      tile_expert/tile_row0/tile_rows [mtiles_max], tile_count [1]) is built
  *      on the GPU by qmoe_tiles_from_ends or qmoe_route_group. */
 int qmoe_gemm_tile_rows(void);
-/* Row-tile sizes the grouped GEMMs take: qmoe_gemm_tile_rows() or 12 (the
+/* Row-tile sizes the grouped GEMMs take: qmoe_gemm_tile_rows(), 32, or 12 (the
  * few-rows kernel, for shapes these return it for). The size to build the
  * tables with for R rows over E experts: one GEMM [K, N], or the expert block
  * (both GEMMs, hidden H, width MI); pass it on as tile_rows_max. */

@@ -26,7 +26,8 @@
 // q*S' is exact). Each lane feeds four 16x16x32 MFMA B fragments per step.
 //
 // Tile: up to 128 rows (8 MFMA row tiles; tiles past the expert's rows are
-// skipped) x 32 int32 word-columns (256 output or 128 SwiGLU columns) per
+// skipped; up to 32 rows in the mid form, whose smaller LDS slots and registers
+// let four workgroups share a CU) x 32 int32 word-columns (256 output or 128 SwiGLU columns) per
 // workgroup of 4 waves; two workgroups per CU give two waves per SIMD, so
 // one wave's dequantisation runs beside the other's MFMA. Wave w owns tile
 // words 8w..8w+7, lane i taking nibbles 4(i/8)..+3 of word i%8 (mode 1: words
@@ -52,16 +53,20 @@ typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;    // 4 waves; two workgroups per CU, so two waves per SIMD
-constexpr int BM = 128;          // rows per tile
-constexpr int MT = BM / 16;      // MFMA row tiles
+constexpr int BM = 128;          // rows per tile (the large form)
+constexpr int kMidRows = 32;     // rows per tile of the mid form
 constexpr int BK = 32;           // k per MFMA step
 constexpr int KC = 64;           // k per staged chunk
 constexpr int NC = 3;            // ring slots of 64-k chunks in LDS (two chunks in flight)
 constexpr int BWORDS = 32;       // int32 word-columns of B per workgroup tile
-constexpr int A_SLOT = BM * KC * 2;       // 16 KB: A fp16 [128][64]
 constexpr int B_SLOT = KC * BWORDS * 4;   // 8 KB: B words [64][32]
 constexpr int S_SLOT = 2 * BWORDS * 16;   // 1 KB: bf16 scales of the groups of the chunk's two steps
-constexpr int SLOT = A_SLOT + B_SLOT + S_SLOT;
+constexpr int a_slot(int rows) { return rows * KC * 2; }  // 16 KB at 128 rows: A fp16 [128][64]
+constexpr size_t gemm_lds(int rows) {
+  // the mid form's per-row data takes the place of the column maxima (used up by then)
+  return (size_t)NC * (a_slot(rows) + B_SLOT + S_SLOT) + 256 * sizeof(uint32_t) +
+         (rows == kMidRows ? 0 : 4 * rows * sizeof(int));
+}
 
 struct GemmArgs {
   const _Float16* a16;       // fp16 activations (row-scaled by 2^rexp), row stride lda
@@ -167,8 +172,10 @@ struct IntC {
   static constexpr int value = N;
 };
 
-template <int MODE>
-__global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f16_kernel(GemmArgs g) {
+template <int MODE, int BM>
+__global__ __launch_bounds__(kThreads, BM == kMidRows ? 4 : 2) void grouped_gemm_f16_kernel(GemmArgs g) {
+  constexpr int MT = BM / 16;  // MFMA row tiles
+  constexpr int A_SLOT = a_slot(BM), SLOT = A_SLOT + B_SLOT + S_SLOT;
   // LDS: a ring of NC chunks, each B (int4 words [64 k][32 word-columns],
   // XOR-swizzled by k-block), A (fp16 [128 rows][64 k], XOR-swizzled by
   // 16-byte chunk) and the raw bf16 scale rows of the groups of its two
@@ -177,7 +184,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f16_kernel(GemmArgs 
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const int G = g.K / g.gs;
   uint32_t* s_mx = reinterpret_cast<uint32_t*>(lds + NC * SLOT);   // [32 words][8 columns]
-  int* s_erow = reinterpret_cast<int*>(s_mx + 256);                 // [BM] row exponents
+  int* s_erow = reinterpret_cast<int*>(s_mx + (BM == kMidRows ? 0 : 256));  // [BM] row exponents
   int* s_orow = s_erow + BM;                                        // [BM] mode 2: output row
   float* s_wrow = reinterpret_cast<float*>(s_orow + BM);            // [BM] mode 2: routing weight
   uint32_t* s_rmax = reinterpret_cast<uint32_t*>(s_wrow + BM);      // [BM] mode 1: row max |act|
@@ -518,6 +525,7 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f16_kernel(GemmArgs 
       if (c + 2 < nch) chunk(IntC<2>{}, c + 2);
     }
   // ---- per-row data to LDS for the epilogue
+  if constexpr (BM == kMidRows) __syncthreads();  // every wave has read the column maxima
   if (tid < BM) {
     s_erow[tid] = drow < rows ? row_e : 0;
     if (MODE == 2) {
@@ -578,18 +586,21 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_f16_kernel(GemmArgs 
   };
   run(live_c);
   };
-  switch (live) {
-    case 1: body(IntC<1>{}); break;
-    case 2: body(IntC<2>{}); break;
-    case 3: body(IntC<3>{}); break;
-    case 4: body(IntC<4>{}); break;
-    case 5: body(IntC<5>{}); break;
-    case 6: body(IntC<6>{}); break;
-    case 7: body(IntC<7>{}); break;
-    default: body(IntC<8>{}); break;
+  if constexpr (MT == 2) {
+    if (live == 1) body(IntC<1>{});
+    else body(IntC<2>{});
+  } else {
+    switch (live) {
+      case 1: body(IntC<1>{}); break;
+      case 2: body(IntC<2>{}); break;
+      case 3: body(IntC<3>{}); break;
+      case 4: body(IntC<4>{}); break;
+      case 5: body(IntC<5>{}); break;
+      case 6: body(IntC<6>{}); break;
+      case 7: body(IntC<7>{}); break;
+      default: body(IntC<8>{}); break;
+    }
   }
-
-
 }
 
 // Per-row exponent and fp16 copy of bf16 rows: e = exponent that puts
@@ -707,10 +718,10 @@ __global__ __launch_bounds__(1024) void slot_reduce_kernel(const uint16_t* __res
   }
 }
 
-constexpr size_t kGemmLds = (size_t)NC * SLOT + 256 * sizeof(uint32_t) + 4 * BM * sizeof(int);
-static_assert(kGemmLds <= 80 * 1024, "two workgroups per CU");
+static_assert(gemm_lds(BM) <= 80 * 1024, "two workgroups per CU");
+static_assert(gemm_lds(kMidRows) <= 40 * 1024, "four workgroups per CU");
 
-template <int MODE>
+template <int MODE, int BM>
 int launch_gemm(const GemmArgs& a, int mtiles_max, hipStream_t st) {
   // grid: every XCD gets ceil(row tiles / 8) row tiles with all their column tiles
   const long nblk = 8L * ((mtiles_max + 7) / 8) * a.n_ntiles;
@@ -722,15 +733,15 @@ int launch_gemm(const GemmArgs& a, int mtiles_max, hipStream_t st) {
   static bool attr_set[64] = {};
   if (dev < 0 || dev >= 64) return QMOE_EINVAL;
   if (!attr_set[dev]) {
-    err = hipFuncSetAttribute((const void*)grouped_gemm_f16_kernel<MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)kGemmLds);
+    err = hipFuncSetAttribute((const void*)grouped_gemm_f16_kernel<MODE, BM>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds(BM));
     if (err != hipSuccess) return (int)err;
     attr_set[dev] = true;
   }
   GemmArgs b = a;
   b.mtiles_max = mtiles_max;
-  hipLaunchKernelGGL((grouped_gemm_f16_kernel<MODE>), dim3((unsigned)nblk), dim3(kThreads),
-                     kGemmLds, st, b);
+  hipLaunchKernelGGL((grouped_gemm_f16_kernel<MODE, BM>), dim3((unsigned)nblk), dim3(kThreads),
+                     gemm_lds(BM), st, b);
   return (int)hipGetLastError();
 }
 
@@ -787,10 +798,14 @@ extern "C" {
 int qmoe_gemm_tile_rows(void) { return BM; }
 
 // The few-rows kernel up to five rows per expert on average: 2560/640 g64, 512
-// experts, 128 / 256 tokens 303 / 327 us per block against 342 / 363, 3072/768
-// 256 tokens 427 against 487; at 512 tokens (ten rows) 543 against 506.
+// experts, 100 / 256 tokens 271 / 320 us per block, 275 / 325 with 32-row tiles
+// here and 304 / 357 with 128-row ones. 32-row tiles (four workgroups per CU
+// instead of two) up to twenty: 512 tokens 349 against 374 us, 1000 382 against
+// 410, 2048/512 Zipf(1.1) 512 tokens 244 against 256; at 1500 tokens (29 rows)
+// 477 against 450, as experts then split into more tiles.
 int qmoe_gemm_tile_rows_for(int R, int E, int K, int N, int gs) {
-  return (long)R <= 5L * E && w4_few_rows_ok(K, N, gs) ? kFewRowsTile : BM;
+  if ((long)R <= 5L * E && w4_few_rows_ok(K, N, gs)) return kFewRowsTile;
+  return (long)R <= 20L * E ? kMidRows : BM;
 }
 
 int qmoe_moe_tile_rows(int R, int E, int H, int MI, int gs_gu, int gs_dn) {
@@ -804,14 +819,14 @@ int qmoe_grouped_gemm_rows(const void* x, int R, int K, int N, int E, int gs, co
                            const void* tile_count, int mtiles_max, void* y, void* workspace, size_t workspace_bytes,
                            void* stream) {
   if (R < 0 || E < 1 || !gemm_shape_ok(K, N, gs) || !aligned16(x) || !aligned16(y) || !aligned16(scale) ||
-      !aligned16(workspace) || tile_expert == nullptr || (tile_rows_max != BM && tile_rows_max != kFewRowsTile) ||
-      (tile_rows_max != BM && !w4_few_rows_ok(K, N, gs)))
+      !aligned16(workspace) || tile_expert == nullptr || (tile_rows_max != BM && tile_rows_max != kMidRows && tile_rows_max != kFewRowsTile) ||
+      (tile_rows_max == kFewRowsTile && !w4_few_rows_ok(K, N, gs)))
     return QMOE_EINVAL;
   if (R == 0) return 0;
   if (workspace_bytes < qmoe_grouped_gemm_workspace(R, K)) return QMOE_EWORKSPACE;
   if (!buffer_extent_ok((size_t)R * K * 2) || !buffer_extent_ok((size_t)K * N / 2)) return QMOE_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  if (tile_rows_max != BM) {
+  if (tile_rows_max == kFewRowsTile) {
     FewRowsArgs f{};
     f.x = (const uint16_t*)x; f.topk = 1; f.w = (const uint32_t*)w; f.s = (const uint16_t*)scale;
     f.K = K; f.N = N; f.gs = gs; f.tile_expert = (const int*)tile_expert; f.tile_row0 = (const int*)tile_row0;
@@ -829,7 +844,7 @@ int qmoe_grouped_gemm_rows(const void* x, int R, int K, int N, int E, int gs, co
   a.tile_expert = (const int*)tile_expert; a.tile_row0 = (const int*)tile_row0;
   a.tile_rows = (const int*)tile_rows; a.tile_count = (const int*)tile_count; a.R = R;
   a.n_ntiles = host_ceil_div(N, 256); a.y = (uint16_t*)y; a.ldy = N;
-  return launch_gemm<0>(a, mtiles_max, st);
+  return tile_rows_max == kMidRows ? launch_gemm<0, kMidRows>(a, mtiles_max, st) : launch_gemm<0, BM>(a, mtiles_max, st);
 }
 
 int qmoe_grouped_gemm(const void* x, int R, int K, int N, int E, int gs, const void* w, const void* scale,
@@ -867,7 +882,7 @@ int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
   a.a16 = x16; a.lda = K; a.a_bytes = (uint32_t)((size_t)M * K * 2); a.topk = 1; a.rexp = rexp;
   a.w = (const uint32_t*)w; a.s = (const uint16_t*)scale; a.K = K; a.N = N; a.gs = gs;
   a.R = M; a.n_ntiles = host_ceil_div(N, 256); a.y = (uint16_t*)y; a.ldy = N;
-  return launch_gemm<0>(a, host_ceil_div(M, BM), st);
+  return launch_gemm<0, BM>(a, host_ceil_div(M, BM), st);
 }
 
 size_t qmoe_moe_prefill_workspace(int T, int k, int H, int MI) { return prefill_layout(T, k, H, MI).total; }
@@ -889,8 +904,8 @@ int qmoe_moe_experts_grouped_rows(const void* x, int T, int H, int MI, int E, in
   if (T < 1 || k < 1 || k > QMOE_KMAX || E < 1 || !gemm_shape_ok(H, 2 * MI, gs_gu) || !gemm_shape_ok(MI, H, gs_dn) ||
       !aligned16(x) || !aligned16(out) || !aligned16(gu_s) || !aligned16(dn_s) || !aligned16(workspace) ||
       (shared != nullptr && !aligned16(shared)) || tile_expert == nullptr ||
-      (tile_rows_max != BM && tile_rows_max != kFewRowsTile) ||
-      (tile_rows_max != BM && (!w4_few_rows_ok(H, 2 * MI, gs_gu) || !w4_few_rows_ok(MI, H, gs_dn))))
+      (tile_rows_max != BM && tile_rows_max != kMidRows && tile_rows_max != kFewRowsTile) ||
+      (tile_rows_max == kFewRowsTile && (!w4_few_rows_ok(H, 2 * MI, gs_gu) || !w4_few_rows_ok(MI, H, gs_dn))))
     return QMOE_EINVAL;
   const PrefillLayout l = prefill_layout(T, k, H, MI);
   if (workspace_bytes < l.total) return QMOE_EWORKSPACE;
@@ -908,7 +923,7 @@ int qmoe_moe_experts_grouped_rows(const void* x, int T, int H, int MI, int E, in
   int* rexp_a = (int*)(ws + l.rexp_a);
   hipStream_t st = (hipStream_t)stream;
   int rc;
-  if (tile_rows_max != BM) {
+  if (tile_rows_max == kFewRowsTile) {
     FewRowsArgs f{};
     f.x = (const uint16_t*)x; f.perm = (const int64_t*)order; f.topk = k;
     f.w = (const uint32_t*)gu_w; f.s = (const uint16_t*)gu_s; f.K = H; f.N = 2 * MI; f.gs = gs_gu;
@@ -930,7 +945,7 @@ int qmoe_moe_experts_grouped_rows(const void* x, int T, int H, int MI, int E, in
     a.tile_expert = (const int*)tile_expert; a.tile_row0 = (const int*)tile_row0;
     a.tile_rows = (const int*)tile_rows; a.tile_count = (const int*)tile_count; a.R = R;
     a.n_ntiles = host_ceil_div(MI, 128); a.y = act; a.ldy = MI; a.MI = MI;
-    rc = launch_gemm<1>(a, mtiles_max, st);
+    rc = tile_rows_max == kMidRows ? launch_gemm<1, kMidRows>(a, mtiles_max, st) : launch_gemm<1, BM>(a, mtiles_max, st);
     if (rc) return rc;
     rc = launch_rows_to_f16(act, R, MI, rmax, rexp_a, act16, nullptr, 0, st);
     if (rc) return rc;
@@ -938,7 +953,7 @@ int qmoe_moe_experts_grouped_rows(const void* x, int T, int H, int MI, int E, in
     d.a16 = act16; d.lda = MI; d.a_bytes = (uint32_t)((size_t)R * MI * 2); d.perm = (const int64_t*)order; d.topk = k; d.rexp = rexp_a; d.rmax_out = nullptr;
     d.w = (const uint32_t*)dn_w; d.s = (const uint16_t*)dn_s; d.K = MI; d.N = H; d.gs = gs_dn;
     d.n_ntiles = host_ceil_div(H, 256); d.y = prod; d.ldy = H; d.wts = (const uint16_t*)wts;
-    rc = launch_gemm<2>(d, mtiles_max, st);
+    rc = tile_rows_max == kMidRows ? launch_gemm<2, kMidRows>(d, mtiles_max, st) : launch_gemm<2, BM>(d, mtiles_max, st);
     if (rc) return rc;
   }
   // one workgroup row covers a token's H / 8 column groups (whole waves, at most 1024 threads), so no

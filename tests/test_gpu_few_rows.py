@@ -37,7 +37,8 @@ def test_grouped(device, K, N, gs):
     counts = [0, 12, 13, 0, 24, 25, 1, 2] + [0] * 16
     E, R = len(counts), int(np.sum(counts)) + 3
     L = _lib.lib()
-    assert L.qmoe_gemm_tile_rows_for(5 * E, E, K, N, gs) == 12 and L.qmoe_gemm_tile_rows_for(5 * E + 1, E, K, N, gs) == 128
+    assert L.qmoe_gemm_tile_rows_for(5 * E, E, K, N, gs) == 12 and L.qmoe_gemm_tile_rows_for(5 * E + 1, E, K, N, gs) == 32
+    assert L.qmoe_gemm_tile_rows_for(20 * E, E, K, N, gs) == 32 and L.qmoe_gemm_tile_rows_for(20 * E + 1, E, K, N, gs) == 128
     log(f"few rows grouped K={K} N={N} gs={gs}")
     ends = np.cumsum(counts).astype(np.int64)
     x, w, s = bf16_normal((R, K), K), int4_words((E, K, N // 8), N), scales((E, K // gs, N), N + 2)
@@ -49,10 +50,28 @@ def test_grouped(device, K, N, gs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,N,gs", [(64, 288, 64), (512, 64, 128), (320, 1056, 32)])
+def test_grouped_mid(device, K, N, gs):
+    """32-row tiles: experts of 15 to 65 rows, one K chunk, ragged columns."""
+    from qmoe import grouped_matmul
+    counts = [0, 15, 16, 17, 31, 32, 33, 64, 65] + [0] * 12
+    E, R = len(counts), int(np.sum(counts))
+    assert 5 * E < R <= 20 * E
+    ends = np.cumsum(counts).astype(np.int64)
+    x, w, s = bf16_normal((R, K), K), int4_words((E, K, N // 8), N), scales((E, K // gs, N), N + 2)
+    y = grouped_matmul([to_dev(x, device)], [to_dev(w, device)], antiquant_scale=[to_dev(s, device)],
+                       group_list=to_dev(ends, device), split_item=3, group_type=0)[0]
+    torch.cuda.synchronize()
+    assert_rounds_exactly(y, *O.grouped_gemm_exact(x, w, s, ends), f"mid rows grouped K={K} N={N}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,E,H,MI,gs,k,zipf", [
     (5, 64, 512, 192, 64, 10, 0.0),     # a partial 128-column act tile
     (32, 64, 320, 256, 32, 10, 1.5),    # 256-column act tiles, experts of more than 12 rows, ragged H
     (8, 32, 4096, 64, 64, 16, 0.0),     # the longest rows, the largest top-k
+    (70, 64, 512, 192, 64, 10, 0.0),    # 32-row tiles: a partial 128-column act tile
+    (120, 64, 320, 64, 32, 10, 1.5),    # and one K chunk in the down projection, experts of more than 32 rows
 ])
 def test_expert_block_stages(device, T, E, H, MI, gs, k, zipf):
     from qmoe import moe_prefill
