@@ -118,7 +118,12 @@ def check(rc: int, what: str) -> None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Raw handle of the current stream of t's device (read directly: building
+    a Stream object for it took 2.0 us of an 11.5 us projection call)."""
+    i = t.get_device()
+    if i < 0:
+        return torch.cuda.current_stream(t.device).cuda_stream  # raises: not a GPU tensor
+    return torch._C._cuda_getCurrentRawStream(i)
 
 
 def ptr(t) -> int | None:

@@ -24,14 +24,14 @@ BF16 = torch.bfloat16
 
 def _cuda(*ts):
     for t in ts:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError("qmoe ops take device tensors")
 
 
 def _same_device(*ts):
-    dev = ts[0].device
+    dev = ts[0].get_device()
     for t in ts[1:]:
-        if t is not None and t.device != dev:
+        if t is not None and t.get_device() != dev:
             raise RuntimeError("all tensors must be on the same device")
 
 
