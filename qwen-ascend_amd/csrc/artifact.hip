@@ -133,6 +133,71 @@ __global__ __launch_bounds__(kThreads) void lqp_scales_kernel(const int8_t* __re
   }
 }
 
+// The same through LDS, four columns per thread: a workgroup's 256 columns (e, n)
+// are 256 G contiguous bytes of s8, read as 16-byte pieces and laid out with an
+// odd row stride, so the 64 lanes of a read (rows 4 apart) fall in different
+// banks; per group a wave writes 512 bytes of scales. The kernel above has every
+// lane read its own row byte by byte, G apart: 63 us for 655360 columns of 40
+// groups and 26 for 1310720 of 10, this one 31 and 22 (scales alone, 79 and 42
+// MB). N a multiple of 4, s8 and scales 16-byte aligned, s8t 4-byte aligned, and
+// the rows fit LDS.
+constexpr int kScaleCols = 256;
+__global__ __launch_bounds__(kThreads) void lqp_scales_vec_kernel(const int8_t* __restrict__ s8,
+                                                                  const uint16_t* __restrict__ base_f16,
+                                                                  int8_t* __restrict__ s8t,
+                                                                  uint16_t* __restrict__ base_bf,
+                                                                  uint16_t* __restrict__ scales, int E, int N, int G) {
+  extern __shared__ unsigned char rows[];  // [256][G | 1]
+  const int S = G | 1;
+  const size_t i0 = (size_t)blockIdx.x * kScaleCols, total = (size_t)E * N;
+  const int cols = (int)min((size_t)kScaleCols, total - i0);
+  const int bytes = cols * G;  // a multiple of 4
+  const unsigned char* src = reinterpret_cast<const unsigned char*>(s8) + i0 * G;
+  for (int p = threadIdx.x * 16; p < bytes; p += kThreads * 16) {
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (p + 16 <= bytes) {
+      v = *reinterpret_cast<const uint4*>(src + p);
+    } else {
+      uint32_t t[4] = {0u, 0u, 0u, 0u};
+      for (int q = 0; p + 4 * q < bytes; ++q) t[q] = *reinterpret_cast<const uint32_t*>(src + p + 4 * q);
+      v = make_uint4(t[0], t[1], t[2], t[3]);
+    }
+    const uint32_t vv[4] = {v.x, v.y, v.z, v.w};
+    int r = p / G, g = p - r * G;
+#pragma unroll
+    for (int b = 0; b < 16; ++b) {
+      if (p + b < bytes) rows[r * S + g] = (unsigned char)(vv[b >> 2] >> (8 * (b & 3)));
+      if (++g == G) {
+        g = 0;
+        ++r;
+      }
+    }
+  }
+  __syncthreads();
+  const int c = 4 * (threadIdx.x & 63);
+  if (c >= cols) return;
+  const size_t i = i0 + c;
+  const size_t e = i / N, n = i % N;  // the four columns are of one expert
+  float bf[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    bf[j] = round_bf16((float)__builtin_bit_cast(_Float16, base_f16[i + j]));
+    if (base_bf != nullptr && threadIdx.x < 64) base_bf[i + j] = (uint16_t)f32_to_bf16(bf[j]);
+  }
+  for (int g = threadIdx.x >> 6; g < G; g += kThreads / 64) {
+    uint32_t q[4], o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      q[j] = rows[(c + j) * S + g];
+      o[j] = f32_to_bf16((float)(int8_t)q[j] * bf[j]);
+    }
+    if (s8t != nullptr)
+      *reinterpret_cast<uint32_t*>(s8t + ((size_t)g * E + e) * N + n) = q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24);
+    if (scales != nullptr)
+      *reinterpret_cast<uint2*>(scales + (e * G + g) * N + n) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+  }
+}
+
 // Scale cache of the W4A16 container (fnx/engine.py:653-659): scales[e, g, n]
 // = bf16(bf16(s8t[g, e, n]) * base[e, n]). The int8 value is exact in bf16
 // and the product of two bf16 is exact in fp32, so one rounding gives the
@@ -171,6 +236,12 @@ int qmoe_lqp_scales(const void* s8, const void* base_fp16, void* s8t, void* base
                     int G, void* stream) {
   if (E < 1 || N < 1 || G < 1) return QMOE_EINVAL;
   const size_t cols = (size_t)E * N;
+  if (N % 4 == 0 && G <= 255 && ((uintptr_t)s8 & 15) == 0 && ((uintptr_t)scales & 15) == 0 && ((uintptr_t)s8t & 3) == 0) {
+    hipLaunchKernelGGL(lqp_scales_vec_kernel, dim3((unsigned)((cols + kScaleCols - 1) / kScaleCols)), dim3(kThreads),
+                       kScaleCols * (G | 1), (hipStream_t)stream, (const int8_t*)s8, (const uint16_t*)base_fp16,
+                       (int8_t*)s8t, (uint16_t*)base_bf16, (uint16_t*)scales, E, N, G);
+    return (int)hipGetLastError();
+  }
   hipLaunchKernelGGL(lqp_scales_kernel, dim3((unsigned)((cols + kThreads - 1) / kThreads)), dim3(kThreads), 0,
                      (hipStream_t)stream, (const int8_t*)s8, (const uint16_t*)base_fp16, (int8_t*)s8t,
                      (uint16_t*)base_bf16, (uint16_t*)scales, E, N, G);

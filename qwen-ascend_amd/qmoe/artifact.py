@@ -59,24 +59,29 @@ def lqp_to_int4pack(v2o, expert_major=True):
     return w4
 
 
-def lqp_scales(s8, base):
-    """LQP scales int8 [E, N, G] + base fp16 [E, N] -> (s8t int8 [G, E, N],
-    base bf16 [E, N], the bf16 scale cache [E, G, N] = bf16(s8 * base_bf16))
-    (``tools/repack_w4a16.py:71-72``, ``fnx/engine.py:653-659``)."""
+def _run_lqp_scales(s8, base, artifact):
+    """(s8t, base bf16, scale cache); the first two are None unless ``artifact``."""
     s8 = _device_tensor(s8, torch.int8, "s8")
     base = _device_tensor(base, torch.float16, "base")
     if s8.dim() != 3 or base.shape != s8.shape[:2]:
         raise RuntimeError("s8 must be [E, N, G] and base [E, N]")
     E, N, G = s8.shape
     dev = s8.device
-    s8t = torch.empty((G, E, N), dtype=torch.int8, device=dev)
-    base_bf = torch.empty((E, N), dtype=torch.bfloat16, device=dev)
+    s8t = torch.empty((G, E, N), dtype=torch.int8, device=dev) if artifact else None
+    base_bf = torch.empty((E, N), dtype=torch.bfloat16, device=dev) if artifact else None
     scales = torch.empty((E, G, N), dtype=torch.bfloat16, device=dev)
     if s8.numel():
-        rc = _lib.lib().qmoe_lqp_scales(s8.data_ptr(), base.data_ptr(), s8t.data_ptr(), base_bf.data_ptr(),
+        rc = _lib.lib().qmoe_lqp_scales(s8.data_ptr(), base.data_ptr(), _lib.ptr(s8t), _lib.ptr(base_bf),
                                         scales.data_ptr(), E, N, G, _lib.stream_of(s8))
         _lib.check(rc, "lqp_scales")
     return s8t, base_bf, scales
+
+
+def lqp_scales(s8, base):
+    """LQP scales int8 [E, N, G] + base fp16 [E, N] -> (s8t int8 [G, E, N],
+    base bf16 [E, N], the bf16 scale cache [E, G, N] = bf16(s8 * base_bf16))
+    (``tools/repack_w4a16.py:71-72``, ``fnx/engine.py:653-659``)."""
+    return _run_lqp_scales(s8, base, True)
 
 
 def conv_proj(v2o, s8, base, expert_major=False):
@@ -98,7 +103,7 @@ def exp_w4_from_lqp(v2o, s8, base):
     """An expert-major :class:`ExpW4` straight from LQP tensors (the container
     and its bf16 scale cache built on the GPU)."""
     w4 = lqp_to_int4pack(v2o, expert_major=True)
-    _, _, scales = lqp_scales(s8, base)
+    scales = _run_lqp_scales(s8, base, False)[2]  # only the cache is kept
     return ExpW4.from_scales(w4, scales)
 
 

@@ -158,3 +158,26 @@ def test_repack_load_decode(device, tmp_path):
     out_b = moe_decode(x, lg, ref["gate_up_proj"], ref["down_proj"], k)[0]
     torch.cuda.synchronize()
     assert np.array_equal(bits(out_a), bits(out_b))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,N,G", [(1, 4, 1), (3, 100, 40), (5, 258, 7), (2, 260, 255), (2, 260, 256), (7, 1284, 16)])
+def test_lqp_scales_edges(device, E, N, G):
+    """Both kernels (rows through LDS or not), workgroups that span experts and a
+    partial last one, and the outputs that may be left out."""
+    from qmoe import _lib
+    from qmoe.artifact import lqp_scales
+    log(f"lqp_scales edges E={E} N={N} G={G}")
+    r = np.random.default_rng(E + N + G)
+    s8 = r.integers(-128, 128, size=(E, N, G)).astype(np.int8)
+    base = (r.standard_normal((E, N)) * 1e-3).astype(np.float16)
+    sd, bd = torch.from_numpy(s8).to(device), torch.from_numpy(base).to(device)
+    s8t, bb, sc = lqp_scales(sd, bd)
+    only = torch.zeros_like(sc)
+    _lib.check(_lib.lib().qmoe_lqp_scales(sd.data_ptr(), bd.data_ptr(), None, None, only.data_ptr(), E, N, G,
+                                          _lib.stream_of(sd)), "lqp_scales")
+    torch.cuda.synchronize()
+    ref_b = O.f32_to_bf16_bits(base.astype(np.float32))
+    ref = O.f32_to_bf16_bits(s8.astype(np.float32) * O.bf16_bits_to_f32(ref_b)[:, :, None]).transpose(0, 2, 1)
+    assert np.array_equal(s8t.cpu().numpy(), s8.transpose(2, 0, 1))
+    assert np.array_equal(bits(bb), ref_b) and np.array_equal(bits(sc), ref) and np.array_equal(bits(only), ref)
