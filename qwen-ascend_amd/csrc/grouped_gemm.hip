@@ -193,22 +193,27 @@ __global__ __launch_bounds__(kThreads, BM == kMidRows ? 4 : 2) void grouped_gemm
   // block of its XCD: XCD x takes row tiles x, x + 8, x + 16, ... in table
   // order (the table lists them longest first), each with all its column
   // tiles in a row, which share their A rows through the XCD's L2.
-  const int tiles_m = (g.tile_expert != nullptr) ? min(g.tile_count[0], g.mtiles_max) : ceil_div(g.R, BM);
   const int xi = (int)(blockIdx.x >> 3);
   const int rt_local = xi / g.n_ntiles;
   const int nt = xi - rt_local * g.n_ntiles;
   const int mt = 8 * rt_local + (int)(blockIdx.x & 7);
-  if (mt >= tiles_m) return;
-  int e, row0, rows;
+  int e, row0, rows, tiles_m;
   if (g.tile_expert != nullptr) {
-    e = g.tile_expert[mt];
-    row0 = g.tile_row0[mt];
-    rows = g.tile_rows[mt];
+    // the table entry is read beside the count, not after it (one round trip
+    // less in the prologue); past the count it is not used
+    const int at = min(mt, g.mtiles_max - 1);
+    tiles_m = min(g.tile_count[0], g.mtiles_max);
+    e = g.tile_expert[at];
+    row0 = g.tile_row0[at];
+    rows = g.tile_rows[at];
+    asm volatile("" : "+s"(e), "+s"(row0), "+s"(rows), "+s"(tiles_m));  // all loaded before the first is tested
   } else {
+    tiles_m = ceil_div(g.R, BM);
     e = 0;
     row0 = mt * BM;
     rows = min(BM, g.R - row0);
   }
+  if (mt >= tiles_m) return;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;

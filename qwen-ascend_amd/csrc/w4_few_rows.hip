@@ -72,25 +72,30 @@ __global__ __launch_bounds__(64 * WC * WK) void w4_few_rows_kernel(FewRowsArgs g
 
   // ---- tile of this block: XCD x takes row tiles x, x + 8, ... in table order,
   // each with its column tiles in a row
-  const int tiles_m = g.tile_expert != nullptr ? min(g.tile_count[0], g.mtiles_max) : (g.R + ROWS - 1) / ROWS;
-  int mt, nt;
+  // The table entry is read beside the count, not after it (one round trip less
+  // ahead of everything else); past the count it is not used.
+  int mt, nt, tiles_m, e = 0, row0 = 0, rows = 0;
   if (g.tile_expert != nullptr) {
     const int xi = (int)(blockIdx.x >> 3);
     nt = xi % n_ntiles;
     mt = 8 * (xi / n_ntiles) + (int)(blockIdx.x & 7);
+    const int at = min(mt, g.mtiles_max - 1);
+    tiles_m = min(g.tile_count[0], g.mtiles_max);
+    e = g.tile_expert[at];
+    row0 = g.tile_row0[at];
+    rows = g.tile_rows[at];
+    asm volatile("" : "+s"(e), "+s"(row0), "+s"(rows), "+s"(tiles_m));  // all loaded before the first is tested
+    rows = min(ROWS, rows);
   } else {
     // dense: the row tiles of a column tile side by side on one XCD
+    tiles_m = (g.R + ROWS - 1) / ROWS;
     const int b = xcd_remap(blockIdx.x, gridDim.x);
     mt = b % tiles_m;
     nt = b / tiles_m;
+    row0 = mt * ROWS;
+    rows = min(ROWS, g.R - row0);
   }
   if (mt >= tiles_m || nt >= n_ntiles) return;
-  int e = 0, row0 = mt * ROWS, rows = min(ROWS, g.R - row0);
-  if (g.tile_expert != nullptr) {
-    e = g.tile_expert[mt];
-    row0 = g.tile_row0[mt];
-    rows = min(ROWS, g.tile_rows[mt]);
-  }
   if (rows <= 0) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
