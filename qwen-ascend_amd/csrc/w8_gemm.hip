@@ -1012,15 +1012,15 @@ int qmoe_w8a16_gemv(const void* x, const void* w, const void* scale, void* y, in
   if (M < 1 || M > 4 || K < 4 || (K % 4) || N < 16 || (N % 16) || group_size < 4 || (group_size % 4) ||
       (K % group_size) || host_ceil_div(N, kTileCols) >= QMOE_DECODE_MAILBOX_BASE - 1)
     return QMOE_EINVAL;
+  const int L = w8_rows_per_thread(K, N, group_size);
+  const int nslices = host_ceil_div(K, kRowLanes * L);
+  if (nslices > 1 && workspace_bytes < qmoe_w8a16_gemv_workspace(M, K, N)) return QMOE_EWORKSPACE;
   // Two to four rows: the skinny MFMA kernel where it takes the shape (its waves
   // share K, so it needs no second reduction through memory): 8.3 against 11.7
   // to 16.5 us (2048 x 8192), 10.5 against 19.2 (three rows, 4096 x 512). One
   // row stays here: from cold weights 9.0 us against 9.75 (2048 x 8192).
   if (M > 1 && w8_mfma_ok(x, w, M, K, N, group_size))
     return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, (hipStream_t)stream);
-  const int L = w8_rows_per_thread(K, N, group_size);
-  const int nslices = host_ceil_div(K, kRowLanes * L);
-  if (nslices > 1 && workspace_bytes < qmoe_w8a16_gemv_workspace(M, K, N)) return QMOE_EWORKSPACE;
   dim3 grid(host_ceil_div(N, kTileCols), nslices);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, (hipStream_t)stream, (const uint16_t*)x, (const int8_t*)w,

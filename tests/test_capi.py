@@ -52,3 +52,20 @@ def test_host_side_shape_queries():
     assert L.qmoe_w4a16_gemv(None, None, None, None, 1, 2048, 4096, 128, None, 0, None, None) == -1  # no counters
     assert L.qmoe_router_topk(None, None, None, 1, 512, 17, None) == -1
     assert L.qmoe_moe_decode(*([None] * 11), 5, 512, 10, 2048, 512, 128, 128, None, 0, None, None) == -1
+
+
+@pytest.mark.parametrize("R,E,K,N,gs,rows", [
+    (1, 512, 2560, 1280, 64, 12), (5 * 64, 64, 4096, 32, 32, 12), (5 * 64 + 1, 64, 4096, 32, 32, 32),
+    (20 * 64, 64, 512, 64, 128, 32), (20 * 64 + 1, 64, 512, 64, 128, 128),
+    (10, 512, 4160, 64, 32, 32),      # rows too long for the few-rows kernel's LDS
+    (10, 512, 96, 64, 32, 32), (10, 512, 64, 48, 32, 32), (10, 512, 64, 64, 16, 32),  # shapes it does not take
+])
+def test_tile_rows_rule(R, E, K, N, gs, rows):
+    """The row-tile size by rows per expert, and the block's as the larger of its
+    two GEMMs' (every size here is one the grouped entry points take)."""
+    from qmoe import _lib
+    L = _lib.lib()
+    assert L.qmoe_gemm_tile_rows_for(R, E, K, N, gs) == rows
+    for MI in (64, 640, 4096, 4160):
+        both = [L.qmoe_gemm_tile_rows_for(R, E, K, 2 * MI, gs), L.qmoe_gemm_tile_rows_for(R, E, MI, K, 64)]
+        assert L.qmoe_moe_tile_rows(R, E, K, MI, gs, 64) == max(both)
