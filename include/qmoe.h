@@ -42,7 +42,8 @@ size_t qmoe_w4a16_gemm_workspace(int M, int K, int N);
 int qmoe_w4a16_gemm_counters(int M, int K, int N);
 int qmoe_w4a16_gemv(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,
                     int group_size, void* workspace, size_t workspace_bytes, void* counters, void* stream);
-/* M > 4: MFMA GEMM on exact fp16 operands. K % 64 == 0, gs % 32 == 0, K/gs <= 56; the workspace
+/* M > 4: MFMA GEMM on exact fp16 operands (few rows: K split over a workgroup's waves, the rows converted
+ * in LDS). K % 64 == 0, gs % 32 == 0; the workspace
  * (qmoe_w4a16_gemm_mfma_workspace(M, K) bytes) holds the rows in fp16 and their exponents. */
 size_t qmoe_w4a16_gemm_mfma_workspace(int M, int K);
 int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,
@@ -357,15 +358,17 @@ int qmoe_shared_gate(const void* sh, const void* gate, long ldg, void* out, long
  *      y[M,N] = bf16(sum_k x[m,k] * q[k,n] * S[k/gs, n]), fp32 accumulation.
  *      x bf16 [M,K], w int8 [K,N], scale bf16 [K/gs, N], y bf16 [M,N];
  *      N % 16 == 0. */
-/* M <= 4: split-K GEMV; K % 4 == 0, gs % 4 == 0; needs
+/* M <= 4: split-K GEMV (two to four rows: the MFMA kernel that splits K over a
+ * workgroup's waves, where K and gs are multiples of 32); K % 4 == 0, gs % 4 == 0; needs
  * qmoe_w8a16_gemv_workspace() bytes (when K > 64) and
  * qmoe_w8a16_gemv_counters(N) counter slots. */
 size_t qmoe_w8a16_gemv_workspace(int M, int K, int N);
 int qmoe_w8a16_gemv_counters(int N);
 int qmoe_w8a16_gemv(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int group_size,
                     void* workspace, size_t workspace_bytes, void* counters, void* stream);
-/* Any M: bf16 MFMA on 64 x 64 tiles, the group scales applied to per-group
- * sums; K % 32 == 0, gs % 32 == 0. */
+/* Any M: bf16 MFMA (few tiles: K split over a workgroup's waves; else 128 x 128
+ * or 128 x 64 tiles), the group scales applied to per-group sums; K % 32 == 0,
+ * gs % 32 == 0. */
 int qmoe_w8a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,
                          int group_size, void* stream);
 
