@@ -134,8 +134,10 @@ __global__ __launch_bounds__(64 * WC * WK) void w4_few_rows_kernel(FewRowsArgs g
     uint32_t b[8];
     uint32_t s[F / 2];
   };
-  const int g0 = s0 / spg;
-  int lq = s0, lrow = g0 * N * 2, lleft = spg - (s0 - g0 * spg), cleft = lleft;
+  // a wave without steps (s0 == nsteps: fewer steps than slices) loads the last
+  // one, which it does not use: row K is past the last expert's weights
+  const int l0 = min(s0, nsteps - 1), g0 = l0 / spg;
+  int lq = l0, lrow = g0 * N * 2, lleft = spg - (l0 - g0 * spg), cleft = lleft;
   auto load_step = [&](Step& v) {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
