@@ -43,7 +43,8 @@ int qmoe_w4a16_gemm_counters(int M, int K, int N);
 int qmoe_w4a16_gemv(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,
                     int group_size, void* workspace, size_t workspace_bytes, void* counters, void* stream);
 /* M > 4: MFMA GEMM on exact fp16 operands (few rows: K split over a workgroup's waves, the rows converted
- * in LDS). K % 64 == 0, gs % 32 == 0; the workspace
+ * in LDS). Any finite scales: sums that leave the fp32 range on the way are taken again in 64 bits.
+ * K % 64 == 0, gs % 32 == 0; the workspace
  * (qmoe_w4a16_gemm_mfma_workspace(M, K) bytes) holds the rows in fp16 and their exponents. */
 size_t qmoe_w4a16_gemm_mfma_workspace(int M, int K);
 int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,

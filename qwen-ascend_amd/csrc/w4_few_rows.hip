@@ -19,7 +19,12 @@
 // their way. A nibble pair becomes fp16 1024 + u or 1024 + 16 u (u = q + 8) in
 // place, without a shift, by one v_bitop3 (mask, flip of the nibble's top bit,
 // exponent), and q = that - 1032 or / 16 - 72 by one packed fma, exact. A scale
-// group's sums are scaled by S[g, n] in fp32; the result by 2^-er.
+// group's sums are scaled by S[g, n] in fp32; the result by 2^-er. Those sums stay
+// below 2^29 |S|, so only a scale above 2^98 can take them out of the fp32 range
+// while the result, 2^er smaller, is in it: an output whose sum is not finite is
+// summed again from the inputs in 64 bits. No scale made from an int8 and an fp16
+// base is near that, so the range costs one test per four outputs (48 rows, 2048 x
+// 4096: 9.17 against 9.12 us), not a pass over the scales ahead of the weights.
 //
 // Modes: 0 = y rows; 1 = SwiGLU act, the first half of the column blocks the gate
 // and the second half the up columns of the same act columns; 2 = down projection with the routing weight,
@@ -292,42 +297,65 @@ __global__ __launch_bounds__(64 * WC * WK) void w4_few_rows_kernel(FewRowsArgs g
   __syncthreads();
 
   // ---- sums over the waves in order, four columns per thread and item
-  auto total = [&](int row, int c, int ex, float (&o)[4]) {
-    float4 a = *reinterpret_cast<const float4*>(red + (size_t)row * CT + c);
+  // Output columns col .. col + 3 of a row from the inputs, in 64 bits
+  auto resum = [&](int row, int col, float (&o)[4]) {
+    const int p = row0 + row;
+    const uint16_t* xr = g.x + (size_t)(MODE == 1 ? perm_lo[2 * (size_t)p] / g.topk : p) * K;
+    double v[4] = {0., 0., 0., 0.};
+#pragma unroll 4
+    for (int k = 0; k < K; ++k) {
+      const uint32_t word = we[(size_t)k * nw + (col >> 3)] >> (4 * (col & 7));  // col is a multiple of 4
+      const uint16_t* sr = se + (size_t)(k / g.gs) * N + col;
+      const double xk = (double)bf16_to_f32(xr[k]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        v[j] += xk * (double)((int)(word << (28 - 4 * j)) >> 28) * (double)bf16_to_f32(sr[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = (float)v[j];
+  };
+  // tile columns c .. c + 3, which are columns col .. of the weights
+  auto total = [&](int row, int c, int col, bool ok_col, int ex, float (&o)[4]) {
+    float4 b[WK];
+#pragma unroll
+    for (int q = 0; q < WK; ++q) b[q] = *reinterpret_cast<const float4*>(red + ((size_t)q * ROWS + row) * CT + c);
+    __builtin_amdgcn_sched_barrier(0);  // every read on its way before the first sum
+    float4 a = b[0];
 #pragma unroll
     for (int q = 1; q < WK; ++q) {
-      const float4 b = *reinterpret_cast<const float4*>(red + ((size_t)q * ROWS + row) * CT + c);
-      a.x += b.x;
-      a.y += b.y;
-      a.z += b.z;
-      a.w += b.w;
+      a.x += b[q].x;
+      a.y += b[q].y;
+      a.z += b[q].z;
+      a.w += b[q].w;
     }
     o[0] = ldexpf(a.x, -ex);
     o[1] = ldexpf(a.y, -ex);
     o[2] = ldexpf(a.z, -ex);
     o[3] = ldexpf(a.w, -ex);
+    // left the fp32 range (not a padding column, nor a row that holds an infinity or NaN)
+    const bool left = !(fabsf(a.x) + fabsf(a.y) + fabsf(a.z) + fabsf(a.w) < INFINITY);
+    if (__builtin_expect(left, 0) && ok_col && ex != exp_to(0x7f80u, 140)) resum(row, col, o);
   };
   constexpr int C4 = (MODE == 1 ? CA : CT) / 4;
   for (int p = tid; p < rows * C4; p += 64 * NW) {
     const int row = p / C4, c = 4 * (p % C4);
-    const int ex = s_erow[row];
+    const int ex = s_erow[row], col = nt * (MODE == 1 ? CA : CT) + c;
+    const bool in = col < (MODE == 1 ? g.MI : N);
     float v[4];
-    total(row, c, ex, v);
+    total(row, c, col, in, ex, v);
     const uint32_t p01 = pk_bf16(v[0], v[1]), p23 = pk_bf16(v[2], v[3]);
     auto lo = [](uint32_t u) { return __uint_as_float(u << 16); };
     auto hi = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
     if (MODE == 1) {
       float u[4];
-      total(row, CA + c, ex, u);
+      total(row, CA + c, g.MI + col, in, ex, u);
       const uint32_t u01 = pk_bf16(u[0], u[1]), u23 = pk_bf16(u[2], u[3]);
-      const int col = nt * CA + c;
-      if (col < g.MI)
+      if (in)
         *reinterpret_cast<uint2*>(g.y + (size_t)(row0 + row) * g.ldy + col) =
             make_uint2(pk_bf16(silu_f32(lo(p01)) * lo(u01), silu_f32(hi(p01)) * hi(u01)),
                        pk_bf16(silu_f32(lo(p23)) * lo(u23), silu_f32(hi(p23)) * hi(u23)));
     } else {
-      const int col = nt * CT + c;
-      if (col < N) {
+      if (in) {
         if (MODE == 2) {
           const float wv = s_wrow[row];
           *reinterpret_cast<uint2*>(g.y + (size_t)s_orow[row] * g.ldy + col) =

@@ -96,3 +96,55 @@ def test_expert_block_stages(device, T, E, H, MI, gs, k, zipf):
     flo[ref["order"]], fhi[ref["order"]] = lo, hi
     assert_in_interval(pb, flo, fhi, f"T={T} prod")
     assert_bf16_equal(ob, O.weighted_reduce(pb, O.f32_to_bf16_bits(np.ones((T, k), np.float32))), f"T={T} sum")
+
+
+def wide_scales(shape, seed, top):
+    """Scales of 2^90 to 2^top in some groups among ordinary ones, columns of only
+    those, columns without (eight times the largest is still an fp32 value)."""
+    r = np.random.default_rng(seed)
+    s = O.bf16_bits_to_f32(scales(shape, seed))
+    big = np.exp2(r.integers(90, top, size=shape)) * (1 + r.integers(0, 128, size=shape) / 128)
+    share = np.broadcast_to(np.array([0.0, 0.1, 0.5, 1.0])[np.arange(shape[-1]) % 4], shape)
+    return O.f32_to_bf16_bits(np.where(r.random(shape) < share, big, s).astype(np.float32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,gs", [(5, 64, 32, 32), (48, 2048, 416, 128), (300, 576, 8224, 96)])
+def test_dense_wide_scales(device, M, K, N, gs):
+    """Scales with which a row's sums leave the fp32 range and its results do not."""
+    from qmoe import weight_quant_batchmatmul
+    log(f"few rows wide scales dense M={M} K={K} N={N} gs={gs}")
+    x = bf16_normal((M, K), M + K, 2.0 ** -100)
+    x[1] = O.f32_to_bf16_bits(O.bf16_bits_to_f32(x[1]) * np.float32(2.0 ** 60))
+    w, s = int4_words((K, N // 8), K + N), wide_scales((K // gs, N), N + 1, 124)
+    y = weight_quant_batchmatmul(to_dev(x, device), to_dev(w, device), to_dev(s, device), antiquant_group_size=gs)
+    torch.cuda.synchronize()
+    assert_rounds_exactly(y, *O.w4a16_gemm_exact(x, w, s, gs), f"few rows wide scales M={M} K={K} N={N}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,H,MI,gs,k", [(64, 512, 192, 64, 10), (64, 320, 256, 32, 10)])
+def test_expert_block_wide_scales(device, E, H, MI, gs, k):
+    """The same in the block: in the gate and up sums of tiny rows and in the down
+    sums (one act tile width each)."""
+    from qmoe import moe_prefill
+    log(f"few rows wide scales block E={E} H={H} MI={MI}")
+    T = 5 * E // k
+    lay = layer(E, H, MI, gs, T + E)
+    lay["gu_s"] = wide_scales((E, H // gs, 2 * MI), 5, 118)
+    lay["dn_s"][:, :, ::3] = 0x7780 | (lay["dn_s"][:, :, ::3] & 0x7f)  # 2^112 to 2^113
+    gu, dn = layer_dev(lay, device)
+    x, lg = bf16_normal((T, H), 3, 2.0 ** -124), bf16_normal((T, E), 4)
+    out, (idx, w, _, ends, order, _), (act, prod) = moe_prefill(
+        to_dev(x, device), to_dev(lg, device), gu, dn, k, return_routing=True, return_intermediates=True)
+    torch.cuda.synchronize()
+    ref = O.moe_prefill(x, lg, lay["gu_w"], lay["gu_s"], lay["dn_w"], lay["dn_s"], k)
+    assert np.array_equal(idx.cpu().numpy(), ref["idx"])
+    ab, pb = bits(act), bits(prod)
+    ge, ga = O.grouped_gemm_exact(x[ref["order"] // k], lay["gu_w"], lay["gu_s"], ref["ends"])
+    assert_in_interval(ab, *O.swiglu_interval(ge[:, :MI], ga[:, :MI], ge[:, MI:], ga[:, MI:]), f"T={T} act")
+    ye, ya = O.grouped_gemm_exact(ab, lay["dn_w"], lay["dn_s"], ref["ends"])
+    lo, hi = prod_interval(ye, ya, ref["w"].reshape(-1)[ref["order"]])
+    flo, fhi = np.empty_like(lo), np.empty_like(hi)
+    flo[ref["order"]], fhi[ref["order"]] = lo, hi
+    assert_in_interval(pb, flo, fhi, f"T={T} prod")
