@@ -47,6 +47,8 @@ int qmoe_w4a16_gemv(const void* x, const void* w, const void* scale, void* y, in
  * K % 64 == 0, gs % 32 == 0; the workspace
  * (qmoe_w4a16_gemm_mfma_workspace(M, K) bytes) holds the rows in fp16 and their exponents. */
 size_t qmoe_w4a16_gemm_mfma_workspace(int M, int K);
+/* 1 where that GEMM takes the few-rows kernel (which leaves the workspace unused), else 0. */
+int qmoe_w4a16_gemm_few_rows(int M, int K, int N, int group_size);
 int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N,
                          int group_size, void* workspace, size_t workspace_bytes, void* stream);
 

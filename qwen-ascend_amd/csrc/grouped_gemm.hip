@@ -860,6 +860,19 @@ int qmoe_grouped_gemm(const void* x, int R, int K, int N, int E, int gs, const v
                                 mtiles_max, y, workspace, workspace_bytes, stream);
 }
 
+// The few-rows kernel for as many rounds of its 128-column workgroups on the 256
+// CUs as K pays for: the tiled kernel's few workgroups each run all of K, so its
+// time grows with K alone (14 us at K = 256, 45 at 2048), while every round of
+// the few-rows kernel costs 6 to 11 us. Few-rows against tiled us (4096 columns;
+// groups of 32 and 128 the same within 4%): K = 64 one round 7.0 / 10.4, two 12.5 /
+// 10.6; K = 256 two 13.1 / 13.9, three 18.8 / 14.0; K = 512 two 14.6 / 18.5, three
+// 21.2 / 18.6; K = 1024 three 24.4 / 27.5, four 32.0 / 27.9; K = 2048 four 42.8 /
+// 46.1; K = 4096 four 68.7 / 82.0.
+int qmoe_w4a16_gemm_few_rows(int M, int K, int N, int gs) {
+  const int rounds = K >= 2048 ? 4 : K >= 1024 ? 3 : K >= 256 ? 2 : 1;
+  return M > 0 && w4_few_rows_ok(K, N, gs) && (long)host_ceil_div(M, 16) * host_ceil_div(N, 128) <= 256L * rounds;
+}
+
 size_t qmoe_w4a16_gemm_mfma_workspace(int M, int K) { return plain_ws(M > 0 ? M : 1, K); }
 
 int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs,
@@ -870,10 +883,7 @@ int qmoe_w4a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
   if (workspace_bytes < qmoe_w4a16_gemm_mfma_workspace(M, K)) return QMOE_EWORKSPACE;
   if (!buffer_extent_ok((size_t)M * K * 2) || !buffer_extent_ok((size_t)K * N / 2)) return QMOE_EINVAL;
   hipStream_t st = (hipStream_t)stream;
-  // The few-rows kernel up to four rounds of its 128-column workgroups on the
-  // CUs: 2048 x 4096 at 64 rows 11.1 against 31.8 us, at 256 21.5 against 45.2,
-  // at 512 40.2 against 45.2.
-  if (w4_few_rows_ok(K, N, gs) && (long)host_ceil_div(M, 16) * host_ceil_div(N, 128) <= 1024) {
+  if (qmoe_w4a16_gemm_few_rows(M, K, N, gs)) {
     FewRowsArgs f{};
     f.x = (const uint16_t*)x; f.topk = 1; f.w = (const uint32_t*)w; f.s = (const uint16_t*)scale;
     f.K = K; f.N = N; f.gs = gs; f.R = M; f.y = (uint16_t*)y; f.ldy = N;

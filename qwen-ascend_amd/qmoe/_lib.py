@@ -32,6 +32,7 @@ SIGNATURES = {
     "qmoe_w4a16_gemm_counters": (I, [I, I, I]),
     "qmoe_w4a16_gemv": (I, [P, P, P, P, I, I, I, I, P, Z, P, P]),
     "qmoe_w4a16_gemm_mfma_workspace": (Z, [I, I]),
+    "qmoe_w4a16_gemm_few_rows": (I, [I, I, I, I]),
     "qmoe_w4a16_gemm_mfma": (I, [P, P, P, P, I, I, I, I, P, Z, P]),
     "qmoe_moe_decode_workspace": (Z, [I, I, I, I]),
     "qmoe_moe_decode_counters": (I, [I, I, I, I]),

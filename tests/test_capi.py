@@ -69,3 +69,14 @@ def test_tile_rows_rule(R, E, K, N, gs, rows):
     for MI in (64, 640, 4096, 4160):
         both = [L.qmoe_gemm_tile_rows_for(R, E, K, 2 * MI, gs), L.qmoe_gemm_tile_rows_for(R, E, MI, K, 64)]
         assert L.qmoe_moe_tile_rows(R, E, K, MI, gs, 64) == max(both)
+
+
+@pytest.mark.parametrize("K,rounds", [(64, 1), (192, 1), (256, 2), (960, 2), (1024, 3), (1984, 3), (2048, 4), (4096, 4)])
+def test_few_rows_rule(K, rounds):
+    """The dense W4 GEMM's kernel by rounds of workgroups (16 rows x 128 columns, 256
+    at once): more of them only where K is long."""
+    from qmoe import _lib
+    few = _lib.lib().qmoe_w4a16_gemm_few_rows
+    assert few(16 * 8 * rounds, K, 4096, 32) == 1 and few(16 * 8 * rounds + 1, K, 4096, 32) == 0
+    assert few(16, K, 128 * 256 * rounds, 32) == 1 and few(16, K, 128 * 256 * rounds + 32, 32) == 0
+    assert few(5, K, 48, 32) == 0 and few(5, K + 32, 64, 32) == 0 and few(5, 4160, 64, 64) == 0

@@ -98,6 +98,22 @@ def test_expert_block_stages(device, T, E, H, MI, gs, k, zipf):
     assert_bf16_equal(ob, O.weighted_reduce(pb, O.f32_to_bf16_bits(np.ones((T, k), np.float32))), f"T={T} sum")
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,gs", [(64, 32), (256, 64), (1024, 128)])
+@pytest.mark.parametrize("over", [0, 1])
+def test_dense_rule_sides(device, K, gs, over):
+    """Both sides of the dense rule's line: the last row count on the few-rows kernel
+    and the next, on the tiled one."""
+    from qmoe import _lib, weight_quant_batchmatmul
+    N = 4096
+    M = next(m for m in range(16, 4096, 16) if not _lib.lib().qmoe_w4a16_gemm_few_rows(m + 1, K, N, gs)) + over
+    log(f"dense rule M={M} K={K} gs={gs}")
+    x, w, s = bf16_normal((M, K), M + K), int4_words((K, N // 8), K + N), scales((K // gs, N), N + 1)
+    y = weight_quant_batchmatmul(to_dev(x, device), to_dev(w, device), to_dev(s, device), antiquant_group_size=gs)
+    torch.cuda.synchronize()
+    assert_rounds_exactly(y, *O.w4a16_gemm_exact(x, w, s, gs), f"dense rule M={M} K={K}")
+
+
 def wide_scales(shape, seed, top):
     """Scales of 2^90 to 2^top in some groups among ordinary ones, columns of only
     those, columns without (eight times the largest is still an fp32 value)."""
