@@ -802,14 +802,27 @@ extern "C" {
 
 int qmoe_gemm_tile_rows(void) { return BM; }
 
-// The few-rows kernel up to five rows per expert on average: 2560/640 g64, 512
-// experts, 100 / 256 tokens 271 / 320 us per block, 275 / 325 with 32-row tiles
-// here and 304 / 357 with 128-row ones. 32-row tiles (four workgroups per CU
-// instead of two) up to twenty: 512 tokens 349 against 374 us, 1000 382 against
-// 410, 2048/512 Zipf(1.1) 512 tokens 244 against 256; at 1500 tokens (29 rows)
-// 477 against 450, as experts then split into more tiles.
+// The few-rows kernel's 12-row tiles up to five rows per expert on average and 2.8e9
+// multiply-adds (2048/512 at 128 tokens is 2.7e9, 3072/768 at 64 is 3.0e9). They save
+// launches and short chains, about 10 us a block, but the host does not see the
+// routing, and the popular experts of a skewed batch fill many 12-row tiles, each of
+// which unpacks the weights again. So the line is drawn by the work that skew can
+// multiply, not by the average alone. us per block with 12- / 32- / 128-row tiles, 512
+// experts top-10 (gate_up decides: K N twice the down projection's):
+//   2048/512   64 tokens uniform 154 / 156 / 180   Zipf(1.2)  90 /  91 / 105   Zipf(2)  61 /  68 /  76
+//   2048/512  128                185 / 196 / 223              137 / 135 / 152            86 /  84 /  94
+//   2560/640   64                229 / 238 / 265              144 / 139 / 154            85 /  84 /  90
+//   2560/640  256                310 / 318 / 352              278 / 249 / 272           194 / 165 / 163
+//   3072/768   32                217 / 220 / 240              135 / 133 / 153            90 /  91 /  99
+//   3072/768   64                313 / 310 / 349              195 / 187 / 208           118 / 113 / 106
+//   3072/768  128                381 / 396 / 453              259 / 251 / 281           177 / 149 / 149
+// (1024/384 g32, 128 experts top-8, 64 tokens 42 / 53 / 54.)
+// 32-row tiles (four workgroups per CU instead of two) up to twenty rows per expert:
+// 512 tokens 349 against 374 us with 128-row ones, 1000 382 against 410, 2048/512
+// Zipf(1.1) 512 tokens 244 against 256; at 1500 tokens (29 rows) 477 against 450, as
+// experts then split into more tiles.
 int qmoe_gemm_tile_rows_for(int R, int E, int K, int N, int gs) {
-  if ((long)R <= 5L * E && w4_few_rows_ok(K, N, gs)) return kFewRowsTile;
+  if ((long)R <= 5L * E && w4_few_rows_ok(K, N, gs) && (long)R * K * N <= 2800000000L) return kFewRowsTile;
   return (long)R <= 20L * E ? kMidRows : BM;
 }
 

@@ -70,6 +70,7 @@ def test_grouped_mid(device, K, N, gs):
     (5, 64, 512, 192, 64, 10, 0.0),     # a partial 128-column act tile
     (32, 64, 320, 256, 32, 10, 1.5),    # 256-column act tiles, experts of more than 12 rows, ragged H
     (8, 32, 4096, 64, 64, 16, 0.0),     # the longest rows, the largest top-k
+    (51, 128, 512, 192, 64, 10, 2.0),   # routed in two launches, popular experts of several 12-row tiles
     (70, 64, 512, 192, 64, 10, 0.0),    # 32-row tiles: a partial 128-column act tile
     (120, 64, 320, 64, 32, 10, 1.5),    # and one K chunk in the down projection, experts of more than 32 rows
 ])
