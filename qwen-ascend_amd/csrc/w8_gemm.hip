@@ -127,18 +127,18 @@ __global__ __launch_bounds__(kThreads) void w8a16_gemv_kernel(const uint16_t* __
   }
 }
 
-// ---------------------------------------------------------------- many tiles: LDS ring
+// ---------------------------------------------------------------- many tiles, other groups: LDS ring
 //
-// bf16 MFMA 16x16x32 on BM x BN output tiles per workgroup of 4 waves (2 x 2,
-// each (BM/2) x (BN/2): TI x TJ MFMA tiles). K runs in KC-wide chunks (one
-// or two MFMA steps) that stream into a ring of RING LDS slots by
-// buffer-resource global->LDS DMA, RING - 1 chunks ahead: the x rows (16-byte
+// bf16 MFMA 16x16x32 on 128 x 64 output tiles per workgroup of 4 waves (2 x 2,
+// each 64 x 32: 4 x 2 MFMA tiles). K runs in 32-k chunks (one MFMA step) that
+// stream into a ring of four LDS slots by
+// buffer-resource global->LDS DMA, three chunks ahead: the x rows (16-byte
 // pieces of a row stored XOR-swizzled by row, so the 16 rows a fragment
-// read touches fall in different banks), the raw int8 weight rows [KC][BN]
-// (row k in row slot k ^ ((k / 4) % (256 / BN)), so the four rows a
+// read touches fall in different banks), the raw int8 weight rows [32][64]
+// (row k in row slot k ^ ((k / 4) % 4), so the four rows a
 // conversion read touches fall in different banks) and the bf16 scale row of
 // the chunk's group. One chunk ahead of the MFMAs
-// every thread converts a 4 k x CPT block of that chunk's weights to bf16
+// every thread converts a 4 k x 2 block of that chunk's weights to bf16
 // (exact: |q| <= 128 has at most 8 significant bits) into one of two
 // transposed buffers [column][k] (rows padded by 4 elements), so a lane's B
 // fragment (8 consecutive k of one column) is two 8-byte reads; one barrier
@@ -178,23 +178,20 @@ QMOE_DEV uint2 lds_read8_untracked(const void* p) {
   return v;
 }
 
-// The weight fragments of a chunk's two MFMA steps (two per step, 16 columns
-// apart), each read from the converted rows as two 8-byte halves, in one
+// The two weight fragments of a chunk (16 columns apart), each read from the
+// converted rows as two 8-byte halves, in one
 // block that waits for its own reads. An ordinary LDS load here would make
 // the compiler wait for every global->LDS DMA in flight (the chunk just issued
 // included), since it cannot tell which LDS bytes a DMA writes; no DMA writes
 // the converted buffers.
-QMOE_DEV void lds_read_frags4(const void* p0, const void* p1, const void* p2, const void* p3, uint4& f0, uint4& f1,
-                              uint4& f2, uint4& f3) {
+QMOE_DEV void lds_read_frags2(const void* p0, const void* p1, uint4& f0, uint4& f1) {
   auto a = [](const void* p) { return (unsigned)(size_t)(__attribute__((address_space(3))) const char*)p; };
   asm volatile(
-      "ds_read2_b64 %0, %4 offset1:1\n\t"
-      "ds_read2_b64 %1, %5 offset1:1\n\t"
-      "ds_read2_b64 %2, %6 offset1:1\n\t"
-      "ds_read2_b64 %3, %7 offset1:1\n\t"
+      "ds_read2_b64 %0, %2 offset1:1\n\t"
+      "ds_read2_b64 %1, %3 offset1:1\n\t"
       "s_waitcnt lgkmcnt(0)"
-      : "=&v"(f0), "=&v"(f1), "=&v"(f2), "=&v"(f3)
-      : "v"(a(p0)), "v"(a(p1)), "v"(a(p2)), "v"(a(p3))
+      : "=&v"(f0), "=&v"(f1)
+      : "v"(a(p0)), "v"(a(p1))
       : "memory");
 }
 
@@ -203,35 +200,31 @@ struct W8C {
   static constexpr int value = V;
 };
 
-template <int BM_, int BN_, int KC_, int RING_>
-struct W8Tile {
-  static constexpr int BM = BM_, BN = BN_, KC = KC_, RING = RING_;
-  static constexpr int TI = BM / 32, TJ = BN / 32;
-  static constexpr int NS = KC / kBK;                   // MFMA steps per chunk
+struct W8Ring {
+  static constexpr int BM = 128, BN = 64, KC = kBK, RING = 4;
+  static constexpr int TI = BM / 32, TJ = BN / 32;      // MFMA tiles per wave
   static constexpr int PPR = KC / 8;                    // 16-byte pieces per x row and chunk
   static constexpr int A_BYTES = BM * 2 * KC;           // x rows of one chunk
   static constexpr int B_BYTES = KC * BN;               // raw int8 weight rows of one chunk
   static constexpr int S_BYTES = BN * 2;                // bf16 scale row of the chunk's group
   static constexpr int SLOT = A_BYTES + B_BYTES + S_BYTES;
   static constexpr int AQ = A_BYTES / 1024 / 4;         // A DMA instructions per wave and chunk
-  static constexpr int BQ = B_BYTES / 1024;             // B DMA instructions per chunk (1 KB each)
-  static constexpr int BQW = (BQ + 3) / 4;              // ... per wave (waves past BQ repeat the last one)
-  static constexpr int IPC = AQ + BQW + 1;              // DMA instructions per wave and chunk (1: scales)
-  static constexpr int KG = KC / 4;                     // converting threads' k-row groups of 4
-  static constexpr int CG = kThreads / KG;              // ... and their column groups
+  static constexpr int BQ = B_BYTES / 1024;             // B DMA instructions per chunk (waves past them repeat the last one)
+  static constexpr int IPC = AQ + 1 + 1;                // DMA instructions per wave and chunk: x, weights, scales
+  static constexpr int CG = kThreads / (KC / 4);        // converting threads' column groups (k-row groups of 4)
   static constexpr int CPT = BN / CG;                   // weight columns per converting thread
-  static constexpr int RPS = BN >= 256 ? 1 : 256 / BN;  // raw weight rows per sweep of the 64 LDS banks
+  static constexpr int RPS = 256 / BN;                  // raw weight rows per sweep of the 64 LDS banks
   static constexpr int LDK = KC + 4;                    // bf16 per row of the converted weights (8-byte aligned)
   static constexpr int CONV = 2 * BN * LDK * 2;         // two converted weight buffers
   static constexpr int LDS = RING * SLOT + CONV;
-  static_assert(A_BYTES % 4096 == 0 && (CPT == 2 || CPT == 4 || CPT == 8), "tile shape");
+  static_assert(CPT == 2 && BQ <= 4, "a converting thread reads two bytes per row, a wave at most 1 KB of weights");
 };
 
-template <class T>
 __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __restrict__ x,
                                                               const int8_t* __restrict__ w,
                                                               const uint16_t* __restrict__ s,
                                                               uint16_t* __restrict__ y, int M, int K, int N, int gs) {
+  using T = W8Ring;
   constexpr int BM = T::BM, BN = T::BN, KC = T::KC, RING = T::RING;
   constexpr int TI = T::TI, TJ = T::TJ, CPT = T::CPT, PPR = T::PPR, LDK = T::LDK;
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -246,11 +239,11 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
   const int wm = wave >> 1, wn = wave & 1;
   const int i16 = lane & 15, kb = lane >> 4;
   // piece swizzle of x row r: the 16 rows of a fragment read spread over the banks
-  auto swz = [](int r) { return PPR == 4 ? ((r >> 2) & 3) : (r & 7); };
+  auto swz = [](int r) { return (r >> 2) & 3; };
 
   // ---- DMA sources. A instruction q of wave w: rows (64 / PPR) (4q + w) +
   // lane / PPR, LDS piece lane % PPR of the row holding k-piece
-  // (lane % PPR) ^ swz(row). B instruction b: 1 KB of the raw [KC][BN] chunk,
+  // (lane % PPR) ^ swz(row). B: wave w takes 1 KB of the raw [KC][BN] chunk,
   // lane l at byte 16 l. Scales: lane l < BN / 32 of wave w fetches 8 columns
   // at w BN / 4 + 8 l of the chunk's group row. Buffer resources bound every
   // access to its tensor; the per-lane offsets are fixed and a wave-uniform
@@ -260,7 +253,7 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, K * N, kRsrcWord3);
   const __amdgpu_buffer_rsrc_t rsrc_s =
       __builtin_amdgcn_make_buffer_rsrc((void*)s, (short)0, (K / gs) * N * 2, kRsrcWord3);
-  uint32_t aoff[T::AQ], boff[T::BQW];
+  uint32_t aoff[T::AQ];
 #pragma unroll
   for (int q = 0; q < T::AQ; ++q) {
     const int r = (64 / PPR) * (4 * q + wave) + lane / PPR;
@@ -270,12 +263,8 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
   // raw weight row k sits in LDS row slot k ^ ((k / 4) % RPS) (an involution):
   // the four rows a converting thread reads at once are then in different banks
   auto row_slot = [](int k) { return k ^ ((k >> 2) & (T::RPS - 1)); };
-#pragma unroll
-  for (int q = 0; q < T::BQW; ++q) {
-    const int b = min(4 * q + wave, T::BQ - 1);
-    const int byte = 1024 * b + 16 * lane;
-    boff[q] = (uint32_t)row_slot(byte / BN) * (uint32_t)N + (uint32_t)(n0 + byte % BN);
-  }
+  const int bblock = min(wave_u, T::BQ - 1), bbyte = 1024 * bblock + 16 * lane;
+  const uint32_t boff = (uint32_t)row_slot(bbyte / BN) * (uint32_t)N + (uint32_t)(n0 + bbyte % BN);
   const uint32_t soff = 2u * (uint32_t)(n0 + wave * (BN / 4) + 8 * (lane & (BN / 32 - 1)));
   auto issue_chunk = [&](int c, int slot) {
     unsigned char* base = lds + slot * T::SLOT;
@@ -284,11 +273,8 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
     for (int q = 0; q < T::AQ; ++q)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(base + (4 * q + wave_u) * 1024),
                                                16, (int)aoff[q], k0 * 2, 0, 0);
-#pragma unroll
-    for (int q = 0; q < T::BQW; ++q)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsrc_b, (__attribute__((address_space(3))) void*)(base + T::A_BYTES + min(4 * q + wave_u, T::BQ - 1) * 1024), 16,
-          (int)boff[q], k0 * N, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rsrc_b, (__attribute__((address_space(3))) void*)(base + T::A_BYTES + bblock * 1024), 16, (int)boff, k0 * N, 0, 0);
     if (lane < BN / 32)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_s,
                                                (__attribute__((address_space(3))) void*)(base + T::A_BYTES + T::B_BYTES + wave_u * (BN / 2)),
@@ -301,32 +287,19 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
   int rawoff[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) rawoff[r] = row_slot(4 * kg + r) * BN + CPT * cg;
-  constexpr int NW = (CPT + 3) / 4;
-  // the raw weight words a thread converts (convert_load), then their bf16
+  // the raw weight bytes a thread converts (convert_load), then their bf16
   // rows written to converted buffer buf (convert_store)
-  auto convert_load = [&](int slot, uint32_t (&rw)[4][NW]) {
+  auto convert_load = [&](int slot, uint32_t (&rw)[4]) {
     const unsigned char* raw = lds + slot * T::SLOT + T::A_BYTES;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const unsigned char* p = raw + rawoff[r];
-      if constexpr (CPT == 8) {
-        const uint2 v = *reinterpret_cast<const uint2*>(p);
-        rw[r][0] = v.x;
-        rw[r][1] = v.y;
-      } else if constexpr (CPT == 4) {
-        rw[r][0] = *reinterpret_cast<const uint32_t*>(p);
-      } else {
-        rw[r][0] = (uint32_t)*reinterpret_cast<const uint16_t*>(p);
-      }
-    }
+    for (int r = 0; r < 4; ++r) rw[r] = (uint32_t)*reinterpret_cast<const uint16_t*>(raw + rawoff[r]);
   };
-  auto convert_store = [&](int buf, const uint32_t (&rw)[4][NW]) {
+  auto convert_store = [&](int buf, const uint32_t (&rw)[4]) {
     uint16_t* dst = sbc + buf * BN * LDK + (CPT * cg) * LDK + 4 * kg;
 #pragma unroll
     for (int cc = 0; cc < CPT; ++cc) {
-      const int wd = cc >> 2, by = cc & 3;
-      const uint32_t lo = i8_to_bf16_bits(rw[0][wd], by) | (i8_to_bf16_bits(rw[1][wd], by) << 16);
-      const uint32_t hi = i8_to_bf16_bits(rw[2][wd], by) | (i8_to_bf16_bits(rw[3][wd], by) << 16);
+      const uint32_t lo = i8_to_bf16_bits(rw[0], cc) | (i8_to_bf16_bits(rw[1], cc) << 16);
+      const uint32_t hi = i8_to_bf16_bits(rw[2], cc) | (i8_to_bf16_bits(rw[3], cc) << 16);
       lds_write8_untracked(dst + cc * LDK, lo, hi);
     }
   };
@@ -353,14 +326,14 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
   else __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   {
-    uint32_t rw[4][NW];
+    uint32_t rw[4];
     convert_load(0, rw);
     convert_store(0, rw);
   }
 
   // one chunk: ring slot SL = c % RING and converted buffer BU = c % 2 are
-  // compile-time constants (the loop below is unrolled over lcm(RING, 2)
-  // chunks), so every LDS address is an immediate offset; FIRST: c starts a
+  // compile-time constants (the loop below is unrolled over RING chunks), so
+  // every LDS address is an immediate offset; FIRST: c starts a
   // scale group, whose first MFMAs take a zero accumulator instead of the
   // group sums being cleared after each group
   auto chunk = [&](auto sl_c, auto bu_c, auto first_c, int c) {
@@ -380,35 +353,28 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (c + RING - 1 < nch) issue_chunk(c + RING - 1, (SL + RING - 1) % RING);
-    // Every LDS read of the chunk goes out together: the raw words of chunk
-    // c + 1 to convert, both steps' weight and activation fragments and, at
-    // the end of a scale group, the group's scale row. Step 0's MFMAs then run
-    // beside the conversion, whose stores precede step 1.
+    // Every LDS read of the chunk goes out together: the raw bytes of chunk
+    // c + 1 to convert, the weight and activation fragments and, at
+    // the end of a scale group, the group's scale row.
     const bool convert_next = c + 1 < nch;
     const bool group_end = (c + 1) % cpg == 0;
-    uint32_t rw[4][NW];
+    uint32_t rw[4];
     if (convert_next) convert_load((SL + 1) % RING, rw);
     const unsigned char* as = lds + SL * T::SLOT;
-    bf16x8_v bf[T::NS][TJ], af[T::NS][TI];
+    bf16x8_v bf[TJ], af[TI];
 #pragma unroll
-    for (int st = 0; st < T::NS; ++st) {
-#pragma unroll
-      for (int i = 0; i < TI; ++i) {
-        const int r = arow[i];
-        af[st][i] = *reinterpret_cast<const bf16x8_v*>(as + r * (2 * KC) + (((4 * st + kb) ^ swz(r)) << 4));
-      }
+    for (int i = 0; i < TI; ++i) {
+      const int r = arow[i];
+      af[i] = *reinterpret_cast<const bf16x8_v*>(as + r * (2 * KC) + ((kb ^ swz(r)) << 4));
     }
     {
-      // weight fragments of both steps (converted rows are 8-byte aligned)
-      static_assert(TJ == 2, "two weight fragments per wave and step");
+      // weight fragments (converted rows are 8-byte aligned)
+      static_assert(TJ == 2, "two weight fragments per wave");
       const uint16_t* bs = sbc + BU * BN * LDK + (wn * (BN / 2) + i16) * LDK + kb * 8;
-      uint4 f[4];
-      lds_read_frags4(bs, bs + 16 * LDK, bs + (T::NS - 1) * kBK, bs + 16 * LDK + (T::NS - 1) * kBK, f[0], f[1], f[2],
-                      f[3]);
-#pragma unroll
-      for (int st = 0; st < T::NS; ++st)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) bf[st][j] = __builtin_bit_cast(bf16x8_v, f[(st ? 2 : 0) + j]);
+      uint4 f0, f1;
+      lds_read_frags2(bs, bs + 16 * LDK, f0, f1);
+      bf[0] = __builtin_bit_cast(bf16x8_v, f0);
+      bf[1] = __builtin_bit_cast(bf16x8_v, f1);
     }
     float sc[TJ];
     if (group_end) {
@@ -418,15 +384,12 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
       for (int j = 0; j < TJ; ++j) sc[j] = col[j] < N ? bf16_to_f32(srow[wn * (BN / 2) + j * 16 + i16]) : 0.f;
     }
 #pragma unroll
-    for (int st = 0; st < T::NS; ++st) {
+    for (int i = 0; i < TI; ++i)
 #pragma unroll
-      for (int i = 0; i < TI; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j)
-          accg[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              af[st][i], bf[st][j], (FIRST && st == 0) ? f32x4_v{0.f, 0.f, 0.f, 0.f} : accg[i][j], 0, 0, 0);
-      if (st == 0 && convert_next) convert_store(1 - BU, rw);
-    }
+      for (int j = 0; j < TJ; ++j)
+        accg[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], FIRST ? f32x4_v{0.f, 0.f, 0.f, 0.f} : accg[i][j],
+                                                             0, 0, 0);
+    if (convert_next) convert_store(1 - BU, rw);
     if (group_end) {
       // end of scale group: acc += S[g, col] * group sums
 #pragma unroll
@@ -441,18 +404,17 @@ __global__ __launch_bounds__(kThreads) void w8a16_mfma_kernel(const uint16_t* __
     if (c % cpg == 0) chunk(sl_c, bu_c, W8C<1>{}, c);
     else chunk(sl_c, bu_c, W8C<0>{}, c);
   };
-  // the loop is unrolled over lcm(RING, 2) chunks
-  constexpr int UN = RING % 2 == 0 ? RING : 2 * RING;
+  static_assert(RING % 2 == 0, "ring slot and converted buffer repeat together");
   auto unrolled = [&](auto self, auto j_c, int c) {
     constexpr int J = decltype(j_c)::value;
-    if constexpr (J < UN) {
+    if constexpr (J < RING) {
       if (c + J < nch) {
-        chunk_at(W8C<J % RING>{}, W8C<J % 2>{}, c + J);
+        chunk_at(W8C<J>{}, W8C<J % 2>{}, c + J);
         self(self, W8C<J + 1>{}, c);
       }
     }
   };
-  for (int c = 0; c < nch; c += UN) unrolled(unrolled, W8C<0>{}, c);
+  for (int c = 0; c < nch; c += RING) unrolled(unrolled, W8C<0>{}, c);
   // D layout: lane holds column i16 of tile (i, j) for rows 4 kb .. 4 kb + 3
 #pragma unroll
   for (int i = 0; i < TI; ++i)
@@ -965,23 +927,23 @@ int launch_w8_reg(const void* x, const void* w, const void* scale, void* y, int 
   return (int)hipGetLastError();
 }
 
-template <class T>
 int launch_w8_mfma(const void* x, const void* w, const void* scale, void* y, int M, int K, int N, int gs,
                    hipStream_t stream) {
+  using T = W8Ring;
   int dev = 0;
   hipError_t err = hipGetDevice(&dev);
   if (err != hipSuccess) return (int)err;
   if (dev < 0 || dev >= 64) return QMOE_EINVAL;
   static bool attr_set[64] = {};
   if (!attr_set[dev]) {
-    err = hipFuncSetAttribute((const void*)w8a16_mfma_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
+    err = hipFuncSetAttribute((const void*)w8a16_mfma_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS);
     if (err != hipSuccess) return (int)err;
     attr_set[dev] = true;
   }
   const long tiles = (long)((M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN);
   const long blocks = (tiles + 7) / 8 * 8;  // whole XCD rounds (extra blocks exit)
   if (blocks > 0x7fffffffL) return QMOE_EINVAL;
-  hipLaunchKernelGGL(w8a16_mfma_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), T::LDS, stream,
+  hipLaunchKernelGGL(w8a16_mfma_kernel, dim3((unsigned)blocks), dim3(kThreads), T::LDS, stream,
                      (const uint16_t*)x, (const int8_t*)w, (const uint16_t*)scale, (uint16_t*)y, M, K, N, gs);
   return (int)hipGetLastError();
 }
@@ -1064,7 +1026,7 @@ int qmoe_w8a16_gemm_mfma(const void* x, const void* w, const void* scale, void* 
   // every CU a workgroup
   if (M <= 256 || (long)host_ceil_div(M, 128) * host_ceil_div(N, 64) < 256)
     return launch_w8_few_tiles(x, w, scale, y, M, K, N, group_size, st);
-  return launch_w8_mfma<W8Tile<128, 64, 32, 4>>(x, w, scale, y, M, K, N, group_size, st);
+  return launch_w8_mfma(x, w, scale, y, M, K, N, group_size, st);
 }
 
 }  // extern "C"

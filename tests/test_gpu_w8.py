@@ -41,8 +41,8 @@ def test_w8a16_gemm(device, M, K, N, gs):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,N,gs", [(512, 2048, 8192, 128), (520, 1024, 6544, 64), (1000, 512, 4160, 128)])
 def test_w8a16_gemm_wide_tiles(device, M, K, N, gs):
-    """Grids of at least 256 128 x 128 tiles (the 8-wave tile), with partial
-    row and column tiles."""
+    """Grids of 256 and a few more 128 x 128 tiles (K split over two groups of
+    waves, and not), with partial row and column tiles."""
     from qmoe import weight_quant_batchmatmul
     log(f"w8a16 wide M={M} K={K} N={N} gs={gs}")
     x, q, S = w8_case(M, K, N, gs, M + 3 * K + N)
@@ -88,6 +88,25 @@ def test_w8a16_register_tiles(device, M, K, N, gs):
     y = weight_quant_batchmatmul(to_dev(x, device), to_dev(q, device), sd, antiquant_group_size=gs)
     torch.cuda.synchronize()
     check(bits(y), x, q, S, gs, f"w8a16 register tiles M={M}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,gs", [
+    (300, 256, 8208, 32), (257, 96, 8208, 32), (300, 32, 8208, 32),  # a group per chunk; three chunks; one
+    (520, 480, 6544, 96), (300, 544, 8208, 544),                     # three chunks per group; one group
+])
+def test_w8a16_ring_tiles(device, M, K, N, gs):
+    """128 x 64 tiles (groups that are not whole 64-k chunks): several scale groups,
+    runs shorter than the ring, partial tiles, scales off a 16-byte boundary."""
+    from qmoe import weight_quant_batchmatmul
+    assert gs % 64 and M > 256 and -(-M // 128) * -(-N // 64) >= 256
+    log(f"w8a16 ring tiles M={M} K={K} N={N} gs={gs}")
+    x, q, S = w8_case(M, K, N, gs, M + K)
+    sd = torch.empty(K // gs * N + 1, dtype=torch.bfloat16, device=device)[1:].view(K // gs, N)
+    sd.copy_(to_dev(S, device))
+    y = weight_quant_batchmatmul(to_dev(x, device), to_dev(q, device), sd, antiquant_group_size=gs)
+    torch.cuda.synchronize()
+    check(bits(y), x, q, S, gs, f"w8a16 ring tiles M={M}")
 
 
 @pytest.mark.gpu
