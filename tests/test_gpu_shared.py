@@ -222,13 +222,9 @@ def test_moe_block_one_token_misaligned_falls_back(device):
     assert _lib.decode_status(_lib.counters(device)) == 0
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("M", [5, 17, 49, 300, 1100])
-@pytest.mark.parametrize("K,MI,rest", [(32, 8, 1), (64, 40, 9), (1536, 100, 300), (256, 1024, 513)])
-def test_bf16_gemm_swiglu(device, M, K, MI, rest):
-    """The fused projection's SwiGLU epilogue over its tile forms (ragged act
-    and rest columns). The operands are whole numbers whose sums are exact in
-    fp32 in any order, so every output bit is determined."""
+def check_gemm_swiglu(device, M, K, MI, rest):
+    """The fused projection with its SwiGLU epilogue. The operands are whole numbers
+    whose sums are exact in fp32 in any order, so every output bit is determined."""
     from qmoe.shared import _gemm
     log(f"bf16 GEMM swiglu M={M} K={K} MI={MI} rest={rest}")
     r = np.random.default_rng(M + K)
@@ -243,3 +239,43 @@ def test_bf16_gemm_swiglu(device, M, K, MI, rest):
     ref, got = O.bf16_bits_to_f32(O.swiglu_bf16(gu, MI)), O.bf16_bits_to_f32(bits(act))
     assert np.all(np.abs(got - ref) <= np.maximum(np.abs(ref) * 2.0 ** -6, 1e-30))
     assert np.mean(got != ref) < 0.01
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [5, 17, 49, 300, 1100])
+@pytest.mark.parametrize("K,MI,rest", [(32, 8, 1), (64, 40, 9), (1536, 100, 300), (256, 1024, 513)])
+def test_bf16_gemm_swiglu(device, M, K, MI, rest):
+    """Ragged act and rest columns from few rows to many."""
+    check_gemm_swiglu(device, M, K, MI, rest)
+
+
+def gemm_form(M, K, MI, rest):
+    """The kernel form the projection takes, by the launch rule: (row tiles, column
+    fragments) with K over 8 or 16 waves, or a tile and its chunk of K."""
+    def up(a, b):
+        return -(-a // b)
+
+    def tiles(bm, bn):
+        return up(M, bm) * (up(MI, bn // 2) + up(rest, bn))
+    for live, f in ((1, 1), (1, 2), (2, 1), (2, 2), (3, 1)):
+        if tiles(16 * live, 16 * f) <= 256:
+            return live, f, 8 if K >= 1536 else 16
+    chunk = 64 if K % 64 == 0 else 32
+    if tiles(64, 64) <= 256:
+        return "64x64", 128 if K % 128 == 0 else chunk
+    return "128x128" if tiles(128, 128) >= 512 else "128x64", chunk
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,MI,rest,form", [
+    (5, 64, 40, 9, (1, 1, 16)), (49, 1536, 100, 300, (1, 1, 8)), (200, 64, 130, 100, (1, 2, 16)),
+    (100, 1536, 400, 100, (1, 2, 8)), (1100, 64, 40, 9, (2, 1, 16)), (1100, 1536, 40, 9, (2, 1, 8)),
+    (100, 64, 500, 300, (2, 2, 16)), (300, 1536, 100, 300, (2, 2, 8)), (4200, 64, 8, 1, (3, 1, 16)),
+    (4200, 1536, 8, 1, (3, 1, 8)), (300, 256, 300, 250, ("64x64", 128)), (300, 192, 300, 250, ("64x64", 64)),
+    (300, 96, 300, 250, ("64x64", 32)), (1100, 64, 500, 100, ("128x64", 64)), (1100, 96, 500, 100, ("128x64", 32)),
+    (2100, 64, 1900, 200, ("128x128", 64)), (2100, 96, 1900, 200, ("128x128", 32)),
+])
+def test_bf16_gemm_swiglu_forms(device, M, K, MI, rest, form):
+    """Every form of the kernel, each with ragged rows, act and rest columns."""
+    assert gemm_form(M, K, MI, rest) == form
+    check_gemm_swiglu(device, M, K, MI, rest)

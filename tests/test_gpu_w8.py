@@ -76,6 +76,7 @@ def test_w8a16_few_tiles(device, M, K, N, gs):
     (200, 128, 8208, 64), (257, 64, 8080, 64),      # K split in two; one chunk, ragged rows and columns
     (130, 512, 8192, 128), (640, 384, 8192, 128),   # 2-chunk groups: split and not
     (1000, 768, 2064, 256), (300, 192, 6544, 192),  # longer groups
+    (300, 1024, 6544, 256), (300, 384, 6544, 192),  # and split: the second half starts at a later scale row
 ])
 def test_w8a16_register_tiles(device, M, K, N, gs):
     """128 x 128 tiles with the conversion in registers: each group length, K
