@@ -81,3 +81,18 @@ def test_few_rows_rule(K, rounds):
     assert few(16 * 8 * rounds, K, 4096, 32) == 1 and few(16 * 8 * rounds + 1, K, 4096, 32) == 0
     assert few(16, K, 128 * 256 * rounds, 32) == 1 and few(16, K, 128 * 256 * rounds + 32, 32) == 0
     assert few(5, K, 48, 32) == 0 and few(5, K + 32, 64, 32) == 0 and few(5, 4160, 64, 64) == 0
+
+
+def test_stream_handle_without_the_private_name(monkeypatch):
+    """A torch without the raw-handle function: the public Stream object's handle."""
+    import importlib.util
+    from types import SimpleNamespace
+
+    import torch
+    from qmoe import _lib
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda dev: SimpleNamespace(cuda_stream=(dev, 7)))
+    spec = importlib.util.spec_from_file_location("qmoe_lib_copy", _lib.__file__)
+    copy = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(copy)
+    assert copy.stream_of(SimpleNamespace(get_device=lambda: 1, device="cuda:1")) == ("cuda:1", 7)
