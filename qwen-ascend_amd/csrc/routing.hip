@@ -340,10 +340,14 @@ __global__ __launch_bounds__(64) void route_scatter_kernel(const int64_t* __rest
   }
 }
 
-// Small batches: the whole grouping in one workgroup, and for a few tokens
-// (KPL > 0) the router as well, wave w routing tokens w, w + 16, ... A launch
-// costs more here than its work: the four grouping launches and the router's
-// take 25 us at 23 tokens, this one 9.
+// Small batches: the whole grouping in one workgroup, and for up to a token per
+// wave (KPL > 0) the router as well, wave w routing token w. A launch costs more
+// here than its work. Graph replay, 512 experts top-10: the router's and the four
+// grouping launches take 18.3 us at 5 tokens and 18.7 at 16, all in one 9.8 and
+// 11.0, the router's launch and this one 10.6 and 10.7 (an eager call is bound by
+// its host side, where one launch less counts). A second token per wave doubles
+// the routing rounds that the grouping waits for: 32 tokens top-16 of 520 experts
+// 25.1 us in one launch against 23.2 in five.
 // Wave w owns a contiguous run of flat ids and ranks them in flat order (ballots
 // within a step of 64, an LDS count per expert between steps); the per-wave
 // counts then become each wave's offset within the expert's run, so the order
@@ -351,7 +355,7 @@ __global__ __launch_bounds__(64) void route_scatter_kernel(const int64_t* __rest
 constexpr int kSmallSteps = 8;       // steps of 64 ids per wave, at most
 constexpr int kSmallIds = 64 * 16 * kSmallSteps;
 constexpr int kSmallExperts = 1024;  // one thread per expert
-constexpr int kSmallTokens = 32;     // tokens routed here: two per wave
+constexpr int kSmallTokens = kScanWaves;  // tokens routed here: one per wave
 
 template <int KPL>
 __global__ __launch_bounds__(1024) void route_small_kernel(const uint16_t* __restrict__ logits,
@@ -374,13 +378,13 @@ __global__ __launch_bounds__(1024) void route_small_kernel(const uint16_t* __res
   if constexpr (KPL > 0) {
     __shared__ int s_idx[kScanWaves][QMOE_KMAX];
     __shared__ float s_w[kScanWaves][QMOE_KMAX];
-    for (int t = wave; t < T; t += kScanWaves) {
-      wave_topk_softmax<KPL>(logits + (size_t)t * E, E, k, s_idx[wave], s_w[wave]);
+    if (wave < T) {
+      wave_topk_softmax<KPL>(logits + (size_t)wave * E, E, k, s_idx[wave], s_w[wave]);
       if (lane < k) {
         const int e = s_idx[wave][lane];
-        s_ids[t * k + lane] = e;
-        idx_out[(size_t)t * k + lane] = e;
-        w_out[(size_t)t * k + lane] = (uint16_t)f32_to_bf16(s_w[wave][lane]);
+        s_ids[wave * k + lane] = e;
+        idx_out[(size_t)wave * k + lane] = e;
+        w_out[(size_t)wave * k + lane] = (uint16_t)f32_to_bf16(s_w[wave][lane]);
       }
     }
     __syncthreads();

@@ -79,10 +79,10 @@ def test_route_group_ignores_invalid_ids(device):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("T,E,k,bm", [(1, 512, 10, 12), (17, 40, 8, 12), (32, 1000, 16, 128), (33, 512, 10, 12),
-                                      (819, 64, 10, 12), (820, 64, 10, 128)])
+                                      (16, 512, 10, 12), (16, 1000, 16, 128), (17, 1000, 16, 12), (819, 64, 10, 12), (820, 64, 10, 128)])
 def test_route_tokens(device, T, E, k, bm):
     """Router and grouping in one call, at the edges of the one-workgroup forms
-    (32 tokens, 8192 ids): ids, stable order and the row-tile table."""
+    (16 tokens, 8192 ids): ids, stable order and the row-tile table."""
     from qmoe.ops import route_tokens
     log(f"route_tokens T={T} E={E} k={k} bm={bm}")
     lg = bf16_normal((T, E), T + E)
