@@ -391,16 +391,23 @@ int run_bf16_gemm(const Bf16Args& a, hipStream_t st) {
     if (a.K % 64 == 0) return launch_bf16_gemm<Bf16Tile<64, 64, 64, 4>, SWIGLU>(a, st);
     return launch_bf16_gemm<Bf16Tile<64, 64, 32, 4>, SWIGLU>(a, st);
   }
-  // 128 x 128 tiles where they give every CU two workgroups, else 128 x 64
-  // (3072 x 2049 at 512 rows 25.2 us against 33.4 with 64 x 64). 64-k chunks,
+  // 128 x 128 tiles where they give every CU two workgroups. 64-k chunks,
   // double-buffered at 128 x 128, where K allows (4096 x 3072 x 2048: 650 -> 980
   // TFLOP/s against 32-k chunks in a 4-slot ring: half the barriers and waits
   // per MFMA)
   if ((long)host_ceil_div(a.M, 128) * col_tiles<SWIGLU>(a, 128) >= 512)
     return a.K % 64 == 0 ? launch_bf16_gemm<Bf16Tile<128, 128, 64, 2>, SWIGLU>(a, st)
                          : launch_bf16_gemm<Bf16Tile<128, 128, 32, 4>, SWIGLU>(a, st);
-  return a.K % 64 == 0 ? launch_bf16_gemm<Bf16Tile<128, 64, 64, 3>, SWIGLU>(a, st)
-                       : launch_bf16_gemm<Bf16Tile<128, 64, 32, 4>, SWIGLU>(a, st);
+  // 128 x 64 tiles where they give every CU one, and with fewer where they run
+  // 64-k chunks of a K of 512 or more; else 64 x 64 tiles, two or more per CU. us from
+  // cold operands, 128 x 64 against 64 x 64: 400 x 768 x 3072 9.9 / 10.8, 512 x 640 x 2560
+  // 9.2 / 11.3, 1200 x 1536 x 1500 15.5 / 19.9, 130 x 512 x 6000 8.2 / 8.2; but 768 x 320
+  // x 1500 6.3 / 5.9, 130 x 320 x 6000 6.9 / 6.5, and with 32-k chunks 640 x 672 x 2048 11.1 /
+  // 9.9, 768 x 1632 x 1500 19.3 / 15.4.
+  const bool full = (long)host_ceil_div(a.M, 128) * col_tiles<SWIGLU>(a, 64) >= 256;
+  if (a.K % 64 == 0 && (full || a.K >= 512)) return launch_bf16_gemm<Bf16Tile<128, 64, 64, 3>, SWIGLU>(a, st);
+  return full ? launch_bf16_gemm<Bf16Tile<128, 64, 32, 4>, SWIGLU>(a, st)
+              : launch_bf16_gemm<Bf16Tile<64, 64, 32, 4>, SWIGLU>(a, st);
 }
 
 bool bf16_gemm_ok(const void* x, long ldx, const void* w, long ldy, int M, int K, int N) {

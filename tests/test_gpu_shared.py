@@ -138,6 +138,22 @@ def test_bf16_gemm_strided_rows(device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [
+    (300, 448, 3601), (300, 1056, 3601),    # 64 x 64 tiles, more than one per CU: K below 512, 32-k chunks
+    (300, 512, 3601),                       # as many from K = 512 on: fewer 128 x 64 ones
+    (1100, 96, 1900),                       # 128 x 64 tiles of 32-k chunks
+])
+def test_bf16_linear_tile_rule(device, M, K, N):
+    """Both sides of the lines between 64 x 64 and 128 x 64 tiles."""
+    from qmoe.shared import linear
+    log(f"bf16 tile rule M={M} K={K} N={N}")
+    x, w = bf16_normal((M, K), K + M), bf16_normal((N, K), N, 0.02)
+    y = linear(to_dev(x, device), to_dev(w, device))
+    torch.cuda.synchronize()
+    check_linear(bits(y), x, w, "linear")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("b", [1, 2, 64, 300])
 def test_moe_block_end_to_end(device, b):
     """Shared + router + experts: rel-L2 <= 2e-3 against the oracle's block
@@ -263,7 +279,11 @@ def gemm_form(M, K, MI, rest):
     chunk = 64 if K % 64 == 0 else 32
     if tiles(64, 64) <= 256:
         return "64x64", 128 if K % 128 == 0 else chunk
-    return "128x128" if tiles(128, 128) >= 512 else "128x64", chunk
+    if tiles(128, 128) >= 512:
+        return "128x128", chunk
+    if tiles(128, 64) >= 256 or (chunk == 64 and K >= 512):
+        return "128x64", chunk
+    return "64x64", 32
 
 
 @pytest.mark.gpu
@@ -272,7 +292,9 @@ def gemm_form(M, K, MI, rest):
     (100, 1536, 400, 100, (1, 2, 8)), (1100, 64, 40, 9, (2, 1, 16)), (1100, 1536, 40, 9, (2, 1, 8)),
     (100, 64, 500, 300, (2, 2, 16)), (300, 1536, 100, 300, (2, 2, 8)), (4200, 64, 8, 1, (3, 1, 16)),
     (4200, 1536, 8, 1, (3, 1, 8)), (300, 256, 300, 250, ("64x64", 128)), (300, 192, 300, 250, ("64x64", 64)),
-    (300, 96, 300, 250, ("64x64", 32)), (1100, 64, 500, 100, ("128x64", 64)), (1100, 96, 500, 100, ("128x64", 32)),
+    (300, 96, 300, 250, ("64x64", 32)), (1100, 512, 500, 100, ("128x64", 64)),
+    (1100, 64, 500, 100, ("64x64", 32)), (1100, 96, 900, 100, ("128x64", 32)),
+    (1100, 96, 500, 100, ("64x64", 32)),
     (2100, 64, 1900, 200, ("128x128", 64)), (2100, 96, 1900, 200, ("128x128", 32)),
 ])
 def test_bf16_gemm_swiglu_forms(device, M, K, MI, rest, form):
