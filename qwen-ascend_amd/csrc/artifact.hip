@@ -137,10 +137,13 @@ __global__ __launch_bounds__(kThreads) void lqp_scales_kernel(const int8_t* __re
 // are 256 G contiguous bytes of s8, read as 16-byte pieces and laid out with an
 // odd row stride, so the 64 lanes of a read (rows 4 apart) fall in different
 // banks; per group a wave writes 512 bytes of scales. The kernel above has every
-// lane read its own row byte by byte, G apart: 63 us for 655360 columns of 40
-// groups and 26 for 1310720 of 10, this one 31 and 22 (scales alone, 79 and 42
-// MB). N a multiple of 4, s8 and scales 16-byte aligned, s8t 4-byte aligned, and
-// the rows fit LDS.
+// lane read its own row byte by byte, G apart: with many groups each line is
+// fetched again for later bytes, with few it lasts. 655360 columns of 40 groups 63 us
+// there, 31 here (scales alone). 1310720 columns, there / here: all outputs 11.8 / 14.3
+// with 5 groups, 18.4 / 18.0 with 10, 31.6 / 22.1 with 16; scales alone 14.4 / 16.9 with
+// 10, 16.5 / 18.0 with 12, 31.1 / 20.7 with 16. So this one from 10 groups on, from 16
+// for the scales alone. N a multiple of 4, s8 and scales 16-byte aligned, s8t 4-byte
+// aligned, and the rows fit LDS.
 constexpr int kScaleCols = 256;
 __global__ __launch_bounds__(kThreads) void lqp_scales_vec_kernel(const int8_t* __restrict__ s8,
                                                                   const uint16_t* __restrict__ base_f16,
@@ -236,7 +239,8 @@ int qmoe_lqp_scales(const void* s8, const void* base_fp16, void* s8t, void* base
                     int G, void* stream) {
   if (E < 1 || N < 1 || G < 1) return QMOE_EINVAL;
   const size_t cols = (size_t)E * N;
-  if (N % 4 == 0 && G <= 255 && ((uintptr_t)s8 & 15) == 0 && ((uintptr_t)scales & 15) == 0 && ((uintptr_t)s8t & 3) == 0) {
+  const int min_groups = s8t != nullptr || base_bf16 != nullptr ? 10 : 16;
+  if (N % 4 == 0 && G >= min_groups && G <= 255 && ((uintptr_t)s8 & 15) == 0 && ((uintptr_t)scales & 15) == 0 && ((uintptr_t)s8t & 3) == 0) {
     hipLaunchKernelGGL(lqp_scales_vec_kernel, dim3((unsigned)((cols + kScaleCols - 1) / kScaleCols)), dim3(kThreads),
                        kScaleCols * (G | 1), (hipStream_t)stream, (const int8_t*)s8, (const uint16_t*)base_fp16,
                        (int8_t*)s8t, (uint16_t*)base_bf16, (uint16_t*)scales, E, N, G);

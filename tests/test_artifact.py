@@ -161,7 +161,7 @@ def test_repack_load_decode(device, tmp_path):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("E,N,G", [(1, 4, 1), (3, 100, 40), (5, 258, 7), (2, 260, 255), (2, 260, 256), (7, 1284, 16)])
+@pytest.mark.parametrize("E,N,G", [(1, 4, 1), (3, 100, 9), (3, 100, 10), (3, 260, 15), (3, 100, 40), (5, 258, 7), (2, 260, 255), (2, 260, 256), (7, 1284, 16)])
 def test_lqp_scales_edges(device, E, N, G):
     """Both kernels (rows through LDS or not), workgroups that span experts and a
     partial last one, and the outputs that may be left out."""
