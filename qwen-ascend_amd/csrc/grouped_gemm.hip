@@ -817,13 +817,17 @@ int qmoe_gemm_tile_rows(void) { return BM; }
 //   3072/768   64                313 / 310 / 349              195 / 187 / 208           118 / 113 / 106
 //   3072/768  128                381 / 396 / 453              259 / 251 / 281           177 / 149 / 149
 // (1024/384 g32, 128 experts top-8, 64 tokens 42 / 53 / 54.)
-// 32-row tiles (four workgroups per CU instead of two) up to twenty rows per expert:
-// 512 tokens 349 against 374 us with 128-row ones, 1000 382 against 410, 2048/512
-// Zipf(1.1) 512 tokens 244 against 256; at 1500 tokens (29 rows) 477 against 450, as
-// experts then split into more tiles.
+// 32-row tiles (four workgroups per CU instead of two) up to twenty rows per expert
+// and 4e10 multiply-adds, 32- / 128-row tiles:
+//   2048/512 1024 tokens uniform 268 / 284   Zipf(0.8) 299 / 307   Zipf(1.2) 298 / 309   Zipf(2) 239 / 228
+//   2560/640 1024                388 / 413             435 / 443             442 / 449           355 / 322
+//   3072/768  768                492 / 532             549 / 558             540 / 545           370 / 347
+//   3072/768 1024                525 / 559             591 / 589             610 / 591           473 / 438
+// Beyond Zipf(1.2) the popular experts' many tiles cost up to a tenth more; at 1500
+// tokens (29 rows) 2560/640 uniform 477 / 450.
 int qmoe_gemm_tile_rows_for(int R, int E, int K, int N, int gs) {
   if ((long)R <= 5L * E && w4_few_rows_ok(K, N, gs) && (long)R * K * N <= 2800000000L) return kFewRowsTile;
-  return (long)R <= 20L * E ? kMidRows : BM;
+  return (long)R <= 20L * E && (long)R * K * N <= 40000000000L ? kMidRows : BM;
 }
 
 int qmoe_moe_tile_rows(int R, int E, int H, int MI, int gs_gu, int gs_dn) {

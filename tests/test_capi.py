@@ -58,6 +58,7 @@ def test_host_side_shape_queries():
     (1, 512, 2560, 1280, 64, 12), (5 * 64, 64, 4096, 32, 32, 12), (5 * 64 + 1, 64, 4096, 32, 32, 32),
     (20 * 64, 64, 512, 64, 128, 32), (20 * 64 + 1, 64, 512, 64, 128, 128),
     (854, 512, 2560, 1280, 64, 12), (855, 512, 2560, 1280, 64, 32),  # few rows per expert, but 2.8e9 multiply-adds
+    (8477, 512, 3072, 1536, 64, 32), (8478, 512, 3072, 1536, 64, 128),  # 4e10
     (10, 512, 4160, 64, 32, 32),      # rows too long for the few-rows kernel's LDS
     (10, 512, 96, 64, 32, 32), (10, 512, 64, 48, 32, 32), (10, 512, 64, 64, 16, 32),  # shapes it does not take
 ])
