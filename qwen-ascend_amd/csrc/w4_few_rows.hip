@@ -24,7 +24,8 @@
 // while the result, 2^er smaller, is in it: an output whose sum is not finite is
 // summed again from the inputs in 64 bits. No scale made from an int8 and an fp16
 // base is near that, so the range costs one test per four outputs (48 rows, 2048 x
-// 4096: 9.17 against 9.12 us), not a pass over the scales ahead of the weights.
+// 4096: 9.17 against 9.12 us), not a pass over the scales ahead of the weights. Where
+// every output of that call is summed again it takes 225 us.
 //
 // Modes: 0 = y rows; 1 = SwiGLU act, the first half of the column blocks the gate
 // and the second half the up columns of the same act columns; 2 = down projection with the routing weight,
